@@ -328,7 +328,7 @@ def rope_table(pos0: int, n_pos: int, head_dim: int, theta: float) -> np.ndarray
 
 
 SCHED_FIELDS = 9  # G2B_SCHED_FIELDS
-KERNEL_NAMES = {1: "k_layer", 2: "k_tiles", 3: "k_short", 4: "k_decode_generic"}
+KERNEL_NAMES = {1: "k_layer", 2: "k_tiles", 3: "k_short", 4: "k_decode_generic", 5: "k_wide"}
 
 
 def schedule_dict(shape: Shape, a) -> dict:

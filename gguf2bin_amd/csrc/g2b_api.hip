@@ -80,6 +80,7 @@ struct g2b_ctx {
   int32_t tune_kernel = 0;     // 0 automatic, 1 k_layer only, 2 k_tiles, 3 spanned k_short
   int32_t *span_ctr = nullptr; // k_short's span tickets (zero between launches)
   size_t span_ctr_cap = 0;
+  int32_t occ_wide = 0;           // k_wide workgroups per CU
   int32_t occ_tiles[2] = {0, 0};  // k_tiles workgroups per CU (static, work queue)
 
   // the last decode call's schedule (g2b_ctx_last_schedule)
@@ -253,6 +254,12 @@ int32_t tiles_slots(g2b_ctx *c, bool wq) {
   int32_t &occ = c->occ_tiles[wq ? 1 : 0];
   if (occ <= 0) occ = tiles_blocks_per_cu(c->sh, wq);
   return std::max(1, c->n_cu) * std::max(1, occ);
+}
+
+// Splits of k_wide that the device holds at once (cached).
+int32_t wide_slots(g2b_ctx *c) {
+  if (c->occ_wide <= 0) c->occ_wide = wide_blocks_per_cu(c->sh);
+  return std::max(1, c->n_cu * std::max(1, c->occ_wide) / wide_groups(c->sh));
 }
 
 // Positions per split of a static schedule.  min_len is the shortest split
@@ -443,8 +450,12 @@ int run_layers(g2b_ctx *c, const SeqDev *d_seqs, const SeqDev &one, int32_t n_se
   const size_t nq = (size_t)nh * hd;
   // (k_layer reads q, k and v as 16-byte pieces; other pointers take the
   // generic kernels)
-  const bool fast = decode_fast_available(c->sh) &&
-                    (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v) & 15u) == 0;
+  const bool aligned = (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v) & 15u) == 0;
+  const bool fast = decode_fast_available(c->sh) && aligned;
+  // Shapes without a k_layer (wide GQA groups, many KV heads, head_dim 256):
+  // k_wide, one launch with the same partials.  Its splits keep the generic
+  // kernel's bounds (length, scratch), so a call that either refuses, both do.
+  const bool wide = !decode_fast_available(c->sh) && aligned && wide_available(c->sh);
 
   DecodeParams dp{};
   dp.sh = c->sh;
@@ -596,6 +607,7 @@ int run_layers(g2b_ctx *c, const SeqDev *d_seqs, const SeqDev &one, int32_t n_se
   }
   const int64_t slots = use_wq ? (tiles ? wq_slots : slots_for(c, dp, true))
                         : tiles ? tiles_slots(c, false)
+                        : wide  ? wide_slots(c)
                                 : slots_for(c, dp, false);
   int32_t max_splits;
   if (use_wq) {
@@ -652,7 +664,9 @@ int run_layers(g2b_ctx *c, const SeqDev *d_seqs, const SeqDev &one, int32_t n_se
     // (measured: four staged chunks or eight per-lane wave-steps per wave, four
     // for one layer of one sequence)
     const int32_t ppw = decode_ppw(c->sh, dp.tune_chunk);
-    const int32_t min_len = !fast                ? 64
+    // (k_wide: two tiles per wave; a split is wide_groups workgroups)
+    const int32_t min_len = wide                 ? 2 * wide_round(c->sh)
+                            : !fast              ? 64
                             : tiles             ? 8 * kTilesRows
                             : dp.stage_rows > 0 ? kWavesPerSplit * 4 * dp.stage_rows
                             : one_unit          ? kWavesPerSplit * 4 * ppw
@@ -693,6 +707,9 @@ int run_layers(g2b_ctx *c, const SeqDev *d_seqs, const SeqDev &one, int32_t n_se
       const int32_t trip = kWavesPerSplit * 2 * ppw;
       split_len = std::max(min_len, split_len / trip * trip);
     }
+    if (wide && c->split_override == 0)  // whole rounds of tiles
+      split_len = std::min<int32_t>(kGenericMaxSplit, (split_len + wide_round(c->sh) - 1) /
+                                                          wide_round(c->sh) * wide_round(c->sh));
     max_splits = (max_pos + 1 + split_len - 1) / split_len;
     if (max_splits > splits_per_seq) {  // lengthen the splits to stay within the budget
       split_len = (int32_t)(((int64_t)max_pos + splits_per_seq) / splits_per_seq);
@@ -705,7 +722,7 @@ int run_layers(g2b_ctx *c, const SeqDev *d_seqs, const SeqDev &one, int32_t n_se
   }
   dp.max_splits = max_splits;
   // one split per unit: the decode kernel writes the output, no combine
-  const bool direct = fast && !use_wq && max_splits == 1 && !att;
+  const bool direct = (fast || wide) && !use_wq && max_splits == 1 && !att;
   dp.direct_out = direct ? 1 : 0;
 
 
@@ -719,7 +736,7 @@ int run_layers(g2b_ctx *c, const SeqDev *d_seqs, const SeqDev &one, int32_t n_se
                               (size_t)g2b_splits_per_layer_cap(n_seq) * nh *
                               (size_t)(kPartHead + hd);
     if (int rc = grow(c, &c->part, &c->part_cap, part_floats, part_limit)) return rc;
-    if (!fast) {
+    if (!fast && !wide) {
       const size_t qf = (size_t)n_layers * n_seq * nq;
       if (int rc = grow(c, &c->qrot, &c->qrot_cap, qf, qf)) return rc;
     }
@@ -728,7 +745,7 @@ int run_layers(g2b_ctx *c, const SeqDev *d_seqs, const SeqDev &one, int32_t n_se
   }
   if (dry) return G2B_OK;  // (the buffers this schedule needs exist now)
 
-  if (!fast) {  // generic shapes: append, decode, combine
+  if (!fast && !wide) {  // generic shapes: append, decode, combine
     AppendParams ap{};
     ap.sh = c->sh;
     ap.seqs = d_seqs;
@@ -750,18 +767,26 @@ int run_layers(g2b_ctx *c, const SeqDev *d_seqs, const SeqDev &one, int32_t n_se
   if (tiles) {
     used_fast = 1;
     G2B_HIP(c, launch_tiles(dp, n_layers, c->stream));
+  } else if (wide) {
+    G2B_HIP(c, launch_wide(dp, n_layers, c->stream));
   } else {
     G2B_HIP(c, launch_decode(dp, n_layers, c->stream, fast, &used_fast));
   }
   // (what launch_layer instantiates: staging only with whole 16-byte row
   // pieces; k_tiles always pulls its tiles into LDS by DMA)
   const int32_t staging = tiles ? 1 : used_fast && dp.stage_rows > 0 ? dp.stage_mode : 0;
-  set_sched(c, tiles ? G2B_KERNEL_TILES : used_fast ? G2B_KERNEL_LAYER : G2B_KERNEL_GENERIC,
+  set_sched(c,
+            tiles       ? G2B_KERNEL_TILES
+            : wide      ? G2B_KERNEL_WIDE
+            : used_fast ? G2B_KERNEL_LAYER
+                        : G2B_KERNEL_GENERIC,
             dp.split_len, use_wq ? dp.piece_len : 0, max_splits,
-            use_wq ? slots : (int64_t)max_splits * n_seq * n_layers, direct && used_fast,
+            use_wq ? slots
+                   : (int64_t)max_splits * n_seq * n_layers * (wide ? wide_groups(c->sh) : 1),
+            direct && (used_fast || wide),
             staging, used_fast && !tiles ? decode_chunk(c->sh, dp.tune_chunk) : 0, att != nullptr);
   if (ev1) G2B_HIP(c, hipEventRecord(ev1, c->stream));
-  if (!direct || !used_fast) G2B_HIP(c, launch_combine(dp, n_layers, c->stream));
+  if (!direct || !(used_fast || wide)) G2B_HIP(c, launch_combine(dp, n_layers, c->stream));
   if (use_wq) {
     // this launch dirtied its set; the combine zeroed the other one
     c->wq_dirty[c->wq_set] = std::max<int32_t>(c->wq_dirty[c->wq_set], (int32_t)n_units + 1);

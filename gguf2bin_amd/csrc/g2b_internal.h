@@ -248,6 +248,21 @@ constexpr int kTilesRows = 16;
 bool tiles_available(const ShapeDev &sh);
 hipError_t launch_tiles(const DecodeParams &p, int n_layers, hipStream_t s);
 int tiles_blocks_per_cu(const ShapeDev &sh, bool wq);
+// Shapes neither k_layer nor k_tiles takes, with head_dim 64, 128 or 256 and
+// up to 16 q heads per KV head: k_wide (g2b_wide.h) does RoPE, append and
+// attention with both products on the matrix cores; static splits, partials
+// as k_layer's.
+bool wide_available(const ShapeDev &sh);
+hipError_t launch_wide(const DecodeParams &p, int n_layers, hipStream_t s);
+// Its resident workgroups per CU, the KV-head groups (workgroups) of a split,
+// and the positions a workgroup's waves take per round of tiles.
+int wide_blocks_per_cu(const ShapeDev &sh);
+int wide_groups(const ShapeDev &sh);
+int wide_round(const ShapeDev &sh);
+template <int FMT, int HD>
+hipError_t launch_wide_hd(const DecodeParams &p, int n_layers, hipStream_t s);
+template <int FMT, int HD>
+int wide_occupancy_hd(const ShapeDev &sh);
 // Resident 256-thread decode workgroups per CU for this shape and the
 // k_layer variant DecodeParams' tune_chunk / stage_mode / stage_rows / wq
 // select (occupancy).

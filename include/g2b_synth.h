@@ -71,7 +71,7 @@ int g2b_ctx_tune_kernel(g2b_ctx *ctx, int32_t kernel);
 
 /* The schedule of the last decode call that launched (g2b_attn_layers,
  * g2b_attn_forward and their variants), into out[G2B_SCHED_FIELDS]:
- *   [0] kernel: G2B_KERNEL_LAYER, _TILES, _SHORT or _GENERIC,
+ *   [0] kernel: G2B_KERNEL_LAYER, _TILES, _SHORT, _GENERIC or _WIDE,
  *   [1] positions per split (k_short: per span; 0 under the work queue),
  *   [2] work-queue piece length (0: static splits or spans),
  *   [3] partial slots per (sequence, layer) (splits, spans or queue slots),
@@ -91,6 +91,7 @@ int g2b_ctx_tune_kernel(g2b_ctx *ctx, int32_t kernel);
 #define G2B_KERNEL_TILES 2
 #define G2B_KERNEL_SHORT 3
 #define G2B_KERNEL_GENERIC 4
+#define G2B_KERNEL_WIDE 5
 int g2b_ctx_last_schedule(const g2b_ctx *ctx, int32_t *out);
 
 /* Kernel timing with HIP events on the context's stream: while enabled,
