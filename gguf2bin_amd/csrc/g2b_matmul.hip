@@ -88,7 +88,19 @@ struct BlockRaw {
 
 template <int FMT>
 __device__ __forceinline__ void load_block(BlockRaw<FMT> &r, const uint8_t *p) {
-  load_dwords<BlockRaw<FMT>::N>(p, r.d, r.sh);
+  if constexpr (FMT == 3) {
+    // (a dword-aligned block ends with its fifth dword: a sixth would lie past
+    // the matrix for its last block)
+    uint32_t d[5];
+    load_dwords<5>(p, d, r.sh);
+#pragma unroll
+    for (int i = 0; i < 5; i++) r.d[i] = d[i];
+    const __attribute__((address_space(1))) uint32_t *last =
+        (const __attribute__((address_space(1))) uint32_t *)(((uintptr_t)p + 18) & ~(uintptr_t)3);
+    r.d[5] = *last;
+  } else {
+    load_dwords<BlockRaw<FMT>::N>(p, r.d, r.sh);
+  }
 }
 
 template <int FMT>
