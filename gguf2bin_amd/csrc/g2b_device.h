@@ -12,6 +12,48 @@ namespace g2b {
 
 constexpr float kNegBig = -1.0e30f;  // "no score yet": finite, so m - m == 0
 
+template <int CTRL>
+__device__ __forceinline__ float dpp_f(float x) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), CTRL, 0xF, 0xF, true));
+}
+
+// Sum over aligned groups of N consecutive lanes; every lane of a group ends
+// with the same value (each step adds two equal-order operands).
+template <int N>
+__device__ __forceinline__ float group_sum(float x) {
+  static_assert(N == 1 || N == 2 || N == 4 || N == 8 || N == 16, "group size");
+  if constexpr (N >= 2) x += dpp_f<0xB1>(x);   // quad_perm [1,0,3,2]: lane ^ 1
+  if constexpr (N >= 4) x += dpp_f<0x4E>(x);   // quad_perm [2,3,0,1]: lane ^ 2
+  if constexpr (N >= 8) x += dpp_f<0x141>(x);  // row_half_mirror: other quad of 8
+  if constexpr (N >= 16) x += dpp_f<0x140>(x); // row_mirror: other half of 16
+  return x;
+}
+
+// x of lane ^ S (S = 32 or 16) through gfx950's lane swaps, on the VALU (no
+// LDS traffic).  With both operands x, v_permlane32_swap leaves lanes 0-31 of
+// its second result holding lanes 32-63 of x and lanes 32-63 of its first
+// result holding lanes 0-31; v_permlane16_swap does the same for each pair of
+// 16-lane rows.
+template <int S>
+__device__ __forceinline__ float lanes_xor(float x) {
+  static_assert(S == 32 || S == 16, "swap distance");
+  const uint32_t u = __float_as_uint(x);
+  if constexpr (S == 32) {
+    const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+    return __uint_as_float((threadIdx.x & 32) ? r[0] : r[1]);
+  } else {
+    const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    return __uint_as_float((threadIdx.x & 16) ? r[0] : r[1]);
+  }
+}
+
+// Sum over the wave, in every lane.
+__device__ __forceinline__ float wave_sum(float x) {
+  x = group_sum<16>(x);
+  x += lanes_xor<16>(x);
+  return x + lanes_xor<32>(x);
+}
+
 // Per-sequence descriptor as the kernels read it (32 bytes).
 struct SeqDev {
   int32_t pos;      // new token position; positions 0..pos are attended
@@ -116,7 +158,14 @@ __device__ __forceinline__ float half_bits_to_f32_hw(uint32_t h) {
 // then, if t < n % 4, element 4 * (n / 4) + t; a tree per wave;
 // (w0 + w1) + (w2 + w3).  rmsnorm's sum (l3_math.c:21-37) in another fp32
 // order; one order for every kernel that normalises, so they agree bitwise.
-// STAGE: also xw[i] = x[i] * w[i] for i < 4 * (n / 4) (xw: LDS).
+// STAGE: also x[i] * w[i] into xw (LDS; n a multiple of 32) in gemv_x_piece's
+// order.
+// Where piece p (elements 4p .. 4p + 3) of an x of nb 32-element blocks lies
+// in LDS, in float4s: piece j of every block together, block by block.  The
+// GEMVs' lanes read piece j of consecutive blocks in one instruction, which
+// this order serves from consecutive addresses; as x lies in memory they are
+// 128 bytes apart, on the same four banks.
+__device__ __forceinline__ int gemv_x_piece(int nb, int p) { return (p & 7) * nb + (p >> 3); }
 template <bool STAGE>
 __device__ inline float wg256_sumsq_t(const float *x, int n, float *red, const float *w,
                                       float *xw) {
@@ -143,14 +192,13 @@ __device__ inline float wg256_sumsq_t(const float *x, int n, float *red, const f
       s = fmaf(v[k].w, v[k].w, s);
       if constexpr (STAGE) {
         if (i0 + 256 * k < n4)
-          reinterpret_cast<float4 *>(xw)[i0 + 256 * k] =
+          reinterpret_cast<float4 *>(xw)[gemv_x_piece(n >> 5, i0 + 256 * k)] =
               make_float4(v[k].x * g[k].x, v[k].y * g[k].y, v[k].z * g[k].z, v[k].w * g[k].w);
       }
     }
   }
   if (t < (n & 3)) s = fmaf(x[4 * n4 + t], x[4 * n4 + t], s);
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+  s = wave_sum(s);
   if ((t & 63) == 0) red[t >> 6] = s;
   __syncthreads();
   return (red[0] + red[1]) + (red[2] + red[3]);

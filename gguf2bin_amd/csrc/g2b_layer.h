@@ -33,41 +33,6 @@
 
 namespace g2b {
 
-template <int CTRL>
-__device__ __forceinline__ float dpp_f(float x) {
-  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), CTRL, 0xF, 0xF, true));
-}
-
-// Sum over aligned groups of N consecutive lanes; every lane of a group ends
-// with the same value (each step adds two equal-order operands).
-template <int N>
-__device__ __forceinline__ float group_sum(float x) {
-  static_assert(N == 1 || N == 2 || N == 4 || N == 8 || N == 16, "group size");
-  if constexpr (N >= 2) x += dpp_f<0xB1>(x);   // quad_perm [1,0,3,2]: lane ^ 1
-  if constexpr (N >= 4) x += dpp_f<0x4E>(x);   // quad_perm [2,3,0,1]: lane ^ 2
-  if constexpr (N >= 8) x += dpp_f<0x141>(x);  // row_half_mirror: other quad of 8
-  if constexpr (N >= 16) x += dpp_f<0x140>(x); // row_mirror: other half of 16
-  return x;
-}
-
-// x of lane ^ S (S = 32 or 16) through gfx950's lane swaps, on the VALU (no
-// LDS traffic).  With both operands x, v_permlane32_swap leaves lanes 0-31 of
-// its second result holding lanes 32-63 of x and lanes 32-63 of its first
-// result holding lanes 0-31; v_permlane16_swap does the same for each pair of
-// 16-lane rows.
-template <int S>
-__device__ __forceinline__ float lanes_xor(float x) {
-  static_assert(S == 32 || S == 16, "swap distance");
-  const uint32_t u = __float_as_uint(x);
-  if constexpr (S == 32) {
-    const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-    return __uint_as_float((threadIdx.x & 32) ? r[0] : r[1]);
-  } else {
-    const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-    return __uint_as_float((threadIdx.x & 16) ? r[0] : r[1]);
-  }
-}
-
 __device__ __forceinline__ float i8f(uint32_t w, int byte) {
   return (float)(int8_t)(uint8_t)(w >> (8 * byte));
 }

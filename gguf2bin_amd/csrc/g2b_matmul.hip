@@ -35,6 +35,9 @@ typedef uint32_t gemv_u32x4 __attribute__((ext_vector_type(4)));
 // at dword alignment)
 typedef uint32_t gemv_u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
 
+// four floats at any 4-byte boundary
+typedef float gemv_f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+
 constexpr int kGemvThreads = 256;
 constexpr int kGemvUnroll = 4;  // steps whose loads are in flight together
 constexpr int kGemvGroup = 8;   // blocks per lane in flight (x in LDS or the cache)
@@ -166,32 +169,26 @@ __device__ __forceinline__ float block_dot(const BlockRaw<FMT> &r, const float *
     return ((a0 + a1) + (a2 + a3)) * (16.f * scale_of(r.d[0], r.sh));
   } else {
     // Q4_1 (gguf_dequant's deq_q4_1, l2_codec.c:65-75): byte j holds
-    // elements j (low nibble) and j + 16 (high), each d * q + m.  With the
-    // same signed-nibble converts as Q4_0 (S = sum (q - 8)/16 * x), the
-    // block is 16 d S + (8 d + m) sum x.  (The reference rounds each weight
-    // d*q + m to fp32 before its products; the difference is within one
-    // fp32 rounding of each product, inside the GEMV bound.)
-    float x0 = 0.f, x1 = 0.f;
+    // elements j (low nibble) and j + 16 (high), each d * q + m in one fp32
+    // rounding (d * q is exact), as the reference dequantises it.  (Summed
+    // apart, d * sum q x and m * sum x can cancel to far less than their own
+    // roundings where a weight near 0 meets an outlier of x.)
+    const float d = scale_of(r.d[0], r.sh);
+    const float m = half_bits_to_f32_hw(r.sh ? (r.d[1] & 0xFFFFu) : (r.d[0] >> 16));
 #pragma unroll
     for (int j = 0; j < 4; j++) {
       const uint32_t w =
           r.sh ? __builtin_amdgcn_perm(r.d[j + 2], r.d[j + 1], 0x05040302u) : r.d[j + 1];
-      const uint32_t t = w ^ 0x88888888u;
-      const uint32_t h = t >> 4;
-      a0 = fmaf(nib_f<0>(t), x[4 * j + 0], a0);
-      a1 = fmaf(nib_f<1>(t), x[4 * j + 1], a1);
-      a0 = fmaf(nib_f<2>(t), x[4 * j + 2], a0);
-      a1 = fmaf(nib_f<3>(t), x[4 * j + 3], a1);
-      a2 = fmaf(nib_f<0>(h), x[16 + 4 * j + 0], a2);
-      a3 = fmaf(nib_f<1>(h), x[16 + 4 * j + 1], a3);
-      a2 = fmaf(nib_f<2>(h), x[16 + 4 * j + 2], a2);
-      a3 = fmaf(nib_f<3>(h), x[16 + 4 * j + 3], a3);
-      x0 += (x[4 * j + 0] + x[4 * j + 1]) + (x[4 * j + 2] + x[4 * j + 3]);
-      x1 += (x[16 + 4 * j + 0] + x[16 + 4 * j + 1]) + (x[16 + 4 * j + 2] + x[16 + 4 * j + 3]);
+      const uint32_t lo = w & 0x0F0F0F0Fu, hi = (w >> 4) & 0x0F0F0F0Fu;
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        const float wl = fmaf(d, (float)((lo >> (8 * k)) & 0xFFu), m);
+        const float wh = fmaf(d, (float)((hi >> (8 * k)) & 0xFFu), m);
+        (k & 1 ? a1 : a0) = fmaf(wl, x[4 * j + k], k & 1 ? a1 : a0);
+        (k & 1 ? a3 : a2) = fmaf(wh, x[16 + 4 * j + k], k & 1 ? a3 : a2);
+      }
     }
-    const float d = scale_of(r.d[0], r.sh);
-    const float m = half_bits_to_f32_hw(r.sh ? (r.d[1] & 0xFFFFu) : (r.d[0] >> 16));
-    return fmaf((a0 + a1) + (a2 + a3), 16.f * d, (x0 + x1) * fmaf(8.f, d, m));
+    return (a0 + a1) + (a2 + a3);
   }
 }
 
@@ -231,19 +228,19 @@ __device__ __forceinline__ void wg_silu_mul(const GemvParams &P, float *xs) {
         r.y = (g[k].y / (1.f + expf(-g[k].y))) * u[k].y;
         r.z = (g[k].z / (1.f + expf(-g[k].z))) * u[k].z;
         r.w = (g[k].w / (1.f + expf(-g[k].w))) * u[k].w;
-        reinterpret_cast<float4 *>(xs)[i0 + kGemvThreads * k] = r;
+        reinterpret_cast<float4 *>(xs)[gemv_x_piece(P.nb, i0 + kGemvThreads * k)] = r;
       }
     }
   }
   __syncthreads();
 }
 
-// x[i..i+4) as the rows read it: plain, rmsnorm'd (x * w from LDS, times
-// inv, as rmsnorm's AVX2 loop) or SiLU x up from LDS.  i is a multiple of 4,
-// x 16-byte aligned.
-__device__ __forceinline__ float4 pro_x4(const GemvParams &P, const float *xs, int i, float inv) {
-  if (P.pro == kProNone) return *reinterpret_cast<const float4 *>(P.x + i);
-  float4 v = *reinterpret_cast<const float4 *>(xs + i);
+// Piece j (elements 4j .. 4j + 3) of block b of x as the rows read it, from
+// LDS: plain, rmsnorm'd (x * w, times inv, as rmsnorm's AVX2 loop) or SiLU x
+// up.
+__device__ __forceinline__ float4 staged_x4(const GemvParams &P, const float *xs, int b, int j,
+                                            float inv) {
+  float4 v = reinterpret_cast<const float4 *>(xs)[j * P.nb + b];
   if (P.pro == kProRmsnorm) {
     v.x *= inv;
     v.y *= inv;
@@ -257,14 +254,16 @@ __device__ __forceinline__ float4 pro_x4(const GemvParams &P, const float *xs, i
 // registers, through the prologue.
 template <int LPR, int KB>
 __device__ __forceinline__ void lane_x(const GemvParams &P, const float *xs, int b0, int b_hi,
-                                       float inv, float (&xr)[KB][32]) {
+                                       float inv, float (&xr)[KB][32], bool staged = true) {
 #pragma unroll
   for (int k = 0; k < KB; k++) {
     const int b = b0 + LPR * k;
 #pragma unroll
     for (int j = 0; j < 32; j += 4) {
       float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-      if (b < b_hi) v = pro_x4(P, xs, 32 * b + j, inv);
+      if (b < b_hi)
+        v = staged ? staged_x4(P, xs, b, j / 4, inv)
+                   : *reinterpret_cast<const float4 *>(P.x + 32 * b + j);
       xr[k][j] = v.x;
       xr[k][j + 1] = v.y;
       xr[k][j + 2] = v.z;
@@ -279,7 +278,7 @@ __device__ __forceinline__ void lane_x(const GemvParams &P, const float *xs, int
 // planes once into LDS - dig[b][plane][chunk] (a dword = one plane of four
 // elements), then exps[b] and units[b] (1, or NaN for a block with a
 // non-finite x: its rows' sums are then NaN) - from x as the rows read it
-// (pro_x4), and each lane loads its blocks' planes into registers.  A
+// (staged_x4), and each lane loads its blocks' planes into registers.  A
 // block's sum_j q_j x_j is then four chains of v_dot4_i32_i8 (exact in
 // int32), combined in fp32 and scaled by the fp16 scale and 2^(e-30): about
 // half the VALU operations of the convert-and-FMA form per weight.  x's
@@ -291,7 +290,8 @@ __device__ __forceinline__ void wg_x_digits(const GemvParams &P, const float *xs
   float *units = reinterpret_cast<float *>(exps + nb);
   for (int it = threadIdx.x; it < nb * 8; it += kGemvThreads) {
     const int b = it >> 3, j = it & 7;  // chunk j: elements 4j .. 4j+3 of block b
-    const float4 v = pro_x4(P, xs, 32 * b + 4 * j, inv);
+    const float4 v = P.pro == kProNone ? reinterpret_cast<const float4 *>(P.x)[it]
+                                       : staged_x4(P, xs, b, j, inv);
     float mx = fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)));
     mx = fmaxf(mx, __shfl_xor(mx, 1));
     mx = fmaxf(mx, __shfl_xor(mx, 2));
@@ -394,29 +394,133 @@ __device__ __forceinline__ void seg_store(const GemvParams &P, int row, float ac
     P.out2[row - P.d01] = acc;
 }
 
+// Sum over aligned groups of LPR lanes, in every lane (DPP and lane swaps:
+// VALU moves, where a shuffle each is an LDS round trip).
 template <int LPR>
 __device__ __forceinline__ float lanes_sum(float v) {
-#pragma unroll
-  for (int o = LPR / 2; o > 0; o >>= 1) v += __shfl_xor(v, o);
+  v = group_sum<(LPR < 16 ? LPR : 16)>(v);
+  if constexpr (LPR >= 32) v += lanes_xor<16>(v);
+  if constexpr (LPR >= 64) v += lanes_xor<32>(v);
   return v;
 }
 
-// Q8_0 / Q4_0.  KB > 0: the lane's x blocks (KB of them) live in registers,
-// prepared while the first weights are in flight (the fused forms: LDS of n
-// floats for SiLU x up); with XD (Q8_0) as digit planes (wg_x_digits, after
-// those n floats in LDS); KB == -1: any nb, x staged once per workgroup in
+// Q8_0 / Q4_0 / Q4_1 rows of up to 128 blocks, plain or fused: the lane's x
+// blocks (KB of them) live in registers, brought there through LDS (nb
+// blocks).  A wave takes UN consecutive wave-steps at a time.  Every load is
+// unconditional - rows and blocks past the end read the last ones and count
+// for nothing.
+//
+// Bound by latency up to a few MB: here a launch that does nothing takes 2.5
+// us and one that only reads 2.2 MB 2.9 us, so everything beside the weights'
+// one round trip shows.  2048 x 1024 Q8_0, back to back, weights from HBM:
+// - 4.0 us with each lane loading its own x (32 floats a lane, 128 bytes
+//   apart: every load instruction touches 32 lines) and four wave-steps
+//   computed whether there were rows for them or not;
+// - 3.4 us with x through LDS but loaded after the weights (the wait for x,
+//   in issue order, then waits for the weights too, and staging it begins
+//   when they have landed);
+// - 2.9 us as here: x goes out first and is staged while the weights come.
+// (A wave staging x for itself, without the barrier: 3.2 us; two blocks a lane
+// over half the waves: 3.2; x 16-byte loads by each lane, first: 3.3.)
+template <int FMT, int LPR, int KB, int UN>
+__global__ __launch_bounds__(kGemvThreads) void k_gemv_rows(GemvParams P) {
+  extern __shared__ float xs[];
+  __shared__ float red[kGemvThreads / 64];
+  constexpr int RPS = 64 / LPR;
+  constexpr int BB = block_bytes<FMT>();
+  constexpr int XP = (LPR * KB * 8 + kGemvThreads - 1) / kGemvThreads;  // pieces of x per thread
+  const int lane = threadIdx.x & 63;
+  const int gw =
+      __builtin_amdgcn_readfirstlane(blockIdx.x * (kGemvThreads / 64) + (threadIdx.x >> 6));
+  const int rr = lane / LPR, c = lane % LPR;
+  const int nb = P.nb, n4 = nb * 8;
+  // x, and what the prologue combines it with (x again where there is none)
+  const float *y = P.pro == kProRmsnorm ? P.nw : P.pro == kProSiluMul ? P.x2 : P.x;
+  float4 xv[XP], yv[XP];
+#pragma unroll
+  for (int k = 0; k < XP; k++) {
+    const int p = min((int)threadIdx.x + kGemvThreads * k, n4 - 1);
+    xv[k] = reinterpret_cast<const float4 *>(P.x)[p];
+    const gemv_f32x4_a4 v = *(const __attribute__((address_space(1))) gemv_f32x4_a4 *)(y + 4 * p);
+    yv[k] = make_float4(v.x, v.y, v.z, v.w);
+  }
+  float xr[KB][32];
+  for (int s0 = gw * UN, trip = 0;; s0 += P.n_waves * UN, trip++) {
+    BlockRaw<FMT> raw[UN][KB];
+#pragma unroll
+    for (int u = 0; u < UN; u++) {
+      const uint8_t *wr = seg_row(P, min(min(s0 + u, P.steps - 1) * RPS + rr, P.d - 1));
+#pragma unroll
+      for (int k = 0; k < KB; k++)
+        load_block<FMT>(raw[u][k], wr + (uint32_t)min(c + LPR * k, nb - 1) * BB);
+    }
+    if (trip == 0) {
+      float ss = 0.f;
+#pragma unroll
+      for (int k = 0; k < XP; k++) {
+        const int p = (int)threadIdx.x + kGemvThreads * k;
+        float4 v = xv[k];
+        const float4 w = yv[k];
+        if (P.pro == kProRmsnorm) {
+          // (wg256_sumsq's order: the model's own rmsnorm gives the same sum)
+          if (p < n4) {
+            ss = fmaf(v.x, v.x, ss);
+            ss = fmaf(v.y, v.y, ss);
+            ss = fmaf(v.z, v.z, ss);
+            ss = fmaf(v.w, v.w, ss);
+          }
+          v = make_float4(v.x * w.x, v.y * w.y, v.z * w.z, v.w * w.w);
+        } else if (P.pro == kProSiluMul) {
+          v.x = (v.x / (1.f + expf(-v.x))) * w.x;
+          v.y = (v.y / (1.f + expf(-v.y))) * w.y;
+          v.z = (v.z / (1.f + expf(-v.z))) * w.z;
+          v.w = (v.w / (1.f + expf(-v.w))) * w.w;
+        }
+        if (p < n4) reinterpret_cast<float4 *>(xs)[gemv_x_piece(nb, p)] = v;
+      }
+      float inv = 1.f;
+      if (P.pro == kProRmsnorm) {
+        ss = wave_sum(ss);
+        if (lane == 0) red[threadIdx.x >> 6] = ss;
+      }
+      __syncthreads();
+      if (P.pro == kProRmsnorm)
+        inv = 1.f / sqrtf(((red[0] + red[1]) + (red[2] + red[3])) / (float)P.n + P.eps);
+      lane_x<LPR, KB>(P, xs, c, nb, inv, xr);
+    }
+#pragma unroll
+    for (int u = 0; u < UN; u++) {
+      float acc = 0.f;
+#pragma unroll
+      for (int k = 0; k < KB; k++) {
+        const float v = block_dot<FMT>(raw[u][k], xr[k]);
+        acc += c + LPR * k < nb ? v : 0.f;
+      }
+      acc = lanes_sum<LPR>(acc);
+      const int row = (s0 + u) * RPS + rr;
+      if (c == 0 && row < P.d) seg_store(P, row, acc);
+    }
+    if (s0 + P.n_waves * UN >= P.steps) break;
+  }
+}
+
+// Q8_0 / Q4_0 / Q4_1, other forms.  XD (Q8_0): the lane's x blocks (KB of
+// them) in registers as digit planes (wg_x_digits, in LDS after the nb blocks
+// of x where there is a prologue), prepared while the first weights are in
+// flight;
+// KB == -1: any nb, x staged once per workgroup in
 // LDS; KB == 0: any nb, x read per block through the cache.
 template <int FMT, int LPR, int KB, bool XD = false>
 __global__ __launch_bounds__(kGemvThreads) void k_gemv_q(GemvParams P) {
-  static_assert(!XD || (FMT == 1 && KB > 0), "digit planes: Q8_0 with x in registers");
+  static_assert(XD ? FMT == 1 && KB > 0 : KB <= 0, "x in registers: as digit planes (Q8_0)");
   extern __shared__ float xs[];
   constexpr int RPS = 64 / LPR;  // rows per wave-step
   constexpr int BB = block_bytes<FMT>();
   const int lane = threadIdx.x & 63;
-  const int gw = blockIdx.x * (kGemvThreads / 64) + (threadIdx.x >> 6);
+  const int gw =
+      __builtin_amdgcn_readfirstlane(blockIdx.x * (kGemvThreads / 64) + (threadIdx.x >> 6));
   const int rr = lane / LPR, c = lane % LPR;
   const int nb = P.nb;
-  [[maybe_unused]] float xr[(KB > 0 && !XD) ? KB : 1][32];
   [[maybe_unused]] uint32_t xd[XD ? KB : 1][4][8];
   [[maybe_unused]] int xe[XD ? KB : 1];
   [[maybe_unused]] float xu[XD ? KB : 1];
@@ -462,24 +566,15 @@ __global__ __launch_bounds__(kGemvThreads) void k_gemv_q(GemvParams P) {
         float inv = 1.f;
         if (P.pro == kProSiluMul) wg_silu_mul(P, xs);
         if (P.pro == kProRmsnorm) inv = wg_rms_stage(P, xs);
-        if constexpr (XD) {
-          uint32_t *dig = reinterpret_cast<uint32_t *>(xs + (P.pro != kProNone ? P.n : 0));
-          wg_x_digits(P, xs, inv, dig);
-          lane_xd<LPR, KB>(P, dig, c, xd, xe, xu);
-        } else {
-          lane_x<LPR, KB>(P, xs, c, nb, inv, xr);
-        }
+        uint32_t *dig = reinterpret_cast<uint32_t *>(xs + (P.pro != kProNone ? P.n : 0));
+        wg_x_digits(P, xs, inv, dig);
+        lane_xd<LPR, KB>(P, dig, c, xd, xe, xu);
       }
 #pragma unroll
       for (int u = 0; u < UN; u++) {
         float acc = 0.f;
 #pragma unroll
-        for (int k = 0; k < KB; k++) {
-          if constexpr (XD)
-            acc += block_dot_xd(raw[u][k], xd[k], xe[k], xu[k]);
-          else
-            acc += block_dot<FMT>(raw[u][k], xr[k]);
-        }
+        for (int k = 0; k < KB; k++) acc += block_dot_xd(raw[u][k], xd[k], xe[k], xu[k]);
         acc = lanes_sum<LPR>(acc);
         if (ok[u] && c == 0) seg_store(P, row[u], acc);
       }
@@ -780,7 +875,7 @@ __global__ __launch_bounds__(kGemvThreads) void k_gemv_mma(GemvParams P) {
 // partial sums in LDS.  Workgroups stride over steps of RPS rows.
 template <int FMT, int LPR, int KB>
 __global__ __launch_bounds__(kGemvThreads) void k_gemv_q_split(GemvParams P) {
-  extern __shared__ float xs[];  // the fused SiLU x up: n floats
+  extern __shared__ float xs[];  // x as the rows read it: nb blocks
   constexpr int RPS = 64 / LPR;
   constexpr int BB = block_bytes<FMT>();
   constexpr int NW = kGemvThreads / 64;
@@ -813,7 +908,7 @@ __global__ __launch_bounds__(kGemvThreads) void k_gemv_q_split(GemvParams P) {
       float inv = 1.f;
       if (P.pro == kProSiluMul) wg_silu_mul(P, xs);
       if (P.pro == kProRmsnorm) inv = wg_rms_stage(P, xs);
-      lane_x<LPR, KB>(P, xs, b_lo + c, b_hi, inv, xr);
+      lane_x<LPR, KB>(P, xs, b_lo + c, b_hi, inv, xr, P.pro != kProNone);
     }
 #pragma unroll
     for (int u = 0; u < kGemvUnroll; u++) {
@@ -928,9 +1023,12 @@ __global__ void k_fill_zero(float *out, int32_t n) {
   if (i < n) out[i] = 0.f;
 }
 
-// LDS of the register-x forms: x * w or SiLU x up of the whole of x
-inline size_t pro_lds(const GemvParams &p) {
-  return p.pro != kProNone ? (size_t)p.n * sizeof(float) : 0;
+// LDS of x, x * w or SiLU x up (all blocks); the split and digit-plane forms
+// keep none of it for a plain x
+inline size_t x_lds(const GemvParams &p) { return (size_t)p.nb * 128u; }
+inline size_t pro_lds(const GemvParams &p) { return p.pro != kProNone ? x_lds(p) : 0; }
+inline size_t xd_lds(const GemvParams &p) {
+  return pro_lds(p) + (size_t)p.nb * 34u * 4u;  // + digit planes, exponents, units
 }
 
 // Resident workgroups per CU of a k_gemv_q instance (with or without the
@@ -951,20 +1049,15 @@ int occ_q(size_t lds) {
   return o;
 }
 
-// kb: 1, 2 x in registers, -1 x in LDS, 0 x through the cache; Q8_0 only:
-// 11, 12 x as digit planes in registers (XD, one or two blocks per lane)
+// kb: -1 x in LDS, 0 x through the cache; Q8_0 only: 11, 12 x as digit
+// planes in registers (XD, one or two blocks per lane)
 template <int FMT, int LPR>
 int occ_q_lpr(int kb, size_t lds) {
   if constexpr (FMT == 1 && LPR >= 16) {
     if (kb == 11) return occ_q<FMT, LPR, 1, true>(lds);
     if (kb == 12) return occ_q<FMT, LPR, 2, true>(lds);
   }
-  switch (kb) {
-    case 1: return occ_q<FMT, LPR, 1>(lds);
-    case 2: return occ_q<FMT, LPR, 2>(lds);
-    case -1: return occ_q<FMT, LPR, -1>(lds);
-    default: return occ_q<FMT, LPR, 0>(lds);
-  }
+  return kb < 0 ? occ_q<FMT, LPR, -1>(lds) : occ_q<FMT, LPR, 0>(lds);
 }
 
 template <int FMT>
@@ -985,7 +1078,7 @@ hipError_t launch_q_lpr(const GemvParams &p, int kb, dim3 grid, hipStream_t s) {
   const dim3 blk(kGemvThreads);
   if constexpr (FMT == 1 && LPR >= 16) {
     if (kb == 11 || kb == 12) {
-      const size_t lds = pro_lds(p) + (size_t)p.nb * 34u * 4u;  // + digit planes, exps, units
+      const size_t lds = xd_lds(p);
       if (kb == 11)
         hipLaunchKernelGGL((k_gemv_q<FMT, LPR, 1, true>), grid, blk, lds, s, p);
       else
@@ -993,15 +1086,58 @@ hipError_t launch_q_lpr(const GemvParams &p, int kb, dim3 grid, hipStream_t s) {
       return hipGetLastError();
     }
   }
-  switch (kb) {
-    case 1: hipLaunchKernelGGL((k_gemv_q<FMT, LPR, 1>), grid, blk, pro_lds(p), s, p); break;
-    case 2: hipLaunchKernelGGL((k_gemv_q<FMT, LPR, 2>), grid, blk, pro_lds(p), s, p); break;
-    case -1:
-      hipLaunchKernelGGL((k_gemv_q<FMT, LPR, -1>), grid, blk, (size_t)p.nb * 128u, s, p);
-      break;
-    default: hipLaunchKernelGGL((k_gemv_q<FMT, LPR, 0>), grid, blk, 0, s, p); break;
-  }
+  if (kb < 0)
+    hipLaunchKernelGGL((k_gemv_q<FMT, LPR, -1>), grid, blk, x_lds(p), s, p);
+  else
+    hipLaunchKernelGGL((k_gemv_q<FMT, LPR, 0>), grid, blk, 0, s, p);
   return hipGetLastError();
+}
+
+template <int FMT, int LPR, int KB>
+hipError_t launch_rows_k(GemvParams p, int n_cu, hipStream_t s) {
+  constexpr int wpw = kGemvThreads / 64;
+  p.steps = (p.d + 64 / LPR - 1) / (64 / LPR);
+  static int occ[2] = {0, 0};
+  // One wave-step per wave up to three workgroups per CU, then two at a time:
+  // 3072 rows of 1024 Q8_0 weights 3.1 us either way, 6144 rows 3.7 us in 768
+  // workgroups of single steps, 3.9 us in 384 of pairs.
+  const bool two = p.steps > 3 * wpw * n_cu;
+  int &o = occ[two ? 1 : 0];
+  if (o == 0) {
+    int n = 0;
+    const hipError_t e =
+        two ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_gemv_rows<FMT, LPR, KB, 2>,
+                                                           kGemvThreads, x_lds(p))
+            : hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_gemv_rows<FMT, LPR, KB, 1>,
+                                                           kGemvThreads, x_lds(p));
+    if (e != hipSuccess || n < 1) {
+      (void)hipGetLastError();
+      n = 1;
+    }
+    o = n;
+  }
+  const int per_wg = wpw * (two ? 2 : 1);
+  const int wgs = std::max(1, std::min((p.steps + per_wg - 1) / per_wg, n_cu * o));
+  p.n_waves = wgs * wpw;
+  if (two)
+    hipLaunchKernelGGL((k_gemv_rows<FMT, LPR, KB, 2>), dim3(wgs), dim3(kGemvThreads), x_lds(p), s, p);
+  else
+    hipLaunchKernelGGL((k_gemv_rows<FMT, LPR, KB, 1>), dim3(wgs), dim3(kGemvThreads), x_lds(p), s, p);
+  return hipGetLastError();
+}
+
+template <int FMT>
+hipError_t launch_rows(const GemvParams &p, int lpr, int kb, int n_cu, hipStream_t s) {
+  if (kb == 2) return launch_rows_k<FMT, 64, 2>(p, n_cu, s);
+  switch (lpr) {
+    case 1: return launch_rows_k<FMT, 1, 1>(p, n_cu, s);
+    case 2: return launch_rows_k<FMT, 2, 1>(p, n_cu, s);
+    case 4: return launch_rows_k<FMT, 4, 1>(p, n_cu, s);
+    case 8: return launch_rows_k<FMT, 8, 1>(p, n_cu, s);
+    case 16: return launch_rows_k<FMT, 16, 1>(p, n_cu, s);
+    case 32: return launch_rows_k<FMT, 32, 1>(p, n_cu, s);
+    default: return launch_rows_k<FMT, 64, 1>(p, n_cu, s);
+  }
 }
 
 template <int FMT, int LPR>
@@ -1154,26 +1290,28 @@ hipError_t launch_gemv(GemvParams p, int32_t type, int n_cu, hipStream_t s) {
       hipLaunchKernelGGL((k_gemv_mma<3, 2>), dim3(wgs), dim3(kGemvThreads), lds, s, p);
     return hipGetLastError();
   }
+  // x in registers: rows of up to 128 blocks.  Q8_0 over many rows takes x as
+  // digit planes (the workgroup's digit prologue pays where every wave has
+  // many rows; LPR >= 16 keeps the instances few).
   int lpr = 1;
   while (lpr < p.nb && lpr < 64) lpr *= 2;
   const int kb = (p.nb + lpr - 1) / lpr;
+  const bool xd = fmt == 1 && lpr >= 16 && p.d >= kGemvXdMinRows;
+  if (p.x_vec4 && kb <= 2 && !xd)
+    return fmt == 1   ? launch_rows<1>(p, lpr, kb, n_cu, s)
+           : fmt == 2 ? launch_rows<2>(p, lpr, kb, n_cu, s)
+                      : launch_rows<3>(p, lpr, kb, n_cu, s);
   const int rps = 64 / lpr;
   p.steps = (p.d + rps - 1) / rps;
-  int kbv = !p.x_vec4                     ? 0
-            : kb <= 2                     ? kb
-            : p.nb * 128 <= kGemvMaxXLds ? -1
-                                          : 0;
-  // Q8_0 with x in registers over many rows: x as digit planes (the
-  // workgroup's digit prologue pays where every wave has many rows; LPR >=
-  // 16 keeps the instances few)
-  if (fmt == 1 && kbv > 0 && lpr >= 16 && p.d >= kGemvXdMinRows) kbv += 10;
+  const int kbv = !p.x_vec4                     ? 0
+                  : kb <= 2                     ? kb + 10
+                  : p.nb * 128 <= kGemvMaxXLds ? -1
+                                                : 0;
   // every wave loads the x of its blocks once: at least kGemvMinSteps steps
   // per wave where there are enough, at least 4 waves per CU, at most one
   // resident round of workgroups (a partial second round would leave most
   // of the chip idle at the end)
-  const size_t lds = kbv < 0    ? (size_t)p.nb * 128u
-                     : kbv > 10 ? pro_lds(p) + (size_t)p.nb * 34u * 4u
-                                : pro_lds(p);
+  const size_t lds = kbv > 10 ? xd_lds(p) : kbv != 0 ? x_lds(p) : 0;
   const int occ = fmt == 1   ? occ_q_fmt<1>(lpr, kbv, lds)
                   : fmt == 2 ? occ_q_fmt<2>(lpr, kbv, lds)
                              : occ_q_fmt<3>(lpr, kbv, lds);
