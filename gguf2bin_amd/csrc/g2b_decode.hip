@@ -289,73 +289,117 @@ __global__ __launch_bounds__(kCombineThreads) void k_combine(DecodeParams P, flo
   G2B_COMBINE_OUT;
 }
 
-// k_combine for one unit's many partials (static splits, more than
-// kCombineFewParts of them, at most kCombineThreads): each head's dims in
-// kCombineParts parts, one workgroup per (head, part), so that a workgroup
-// requests R rows of a quarter of the dims instead of a whole head's rows
-// (c1 / c2, 129 partials of 16 heads: 16 workgroups of 17 row loads per
-// thread became 64 of 5).  The same float64 merge as k_combine - weights
-// exp2(m_p - M), sums over the partials in GRP groups, then over the groups
-// in order, divided by the sum of the weighted l - with the partials dealt
-// to more groups, so the order of the float64 additions differs.
-constexpr int kCombineParts = 4;
-template <int R>
+// k_combine for static splits of few units: each head's dims in PARTS parts,
+// one workgroup per (head, part).  The launch is a chain of dependent steps
+// behind the decode kernel (a single sequence's layer is two launches), so:
+// the parameters in one batch of scalar loads, one round of memory loads (each
+// thread R partials' m, l and four dims), one barrier for the maximum, sums
+// over the lanes by lane swaps and one barrier for the rest.  The
+// whole step of 28 layers, against this combine with a block reduction per sum:
+// one sequence, 129 partials of 16 heads, F32 409 -> 369 us, Q8_0 513 -> 473;
+// eight sequences of up to 45 partials, heads of 128 in groups of 8, 619 -> 560;
+// 64 ragged sequences (1024 heads) 872 -> 835.
+// The same float64 merge as k_combine - weights exp2(m_p - M), sums over the
+// partials, divided by the sum of the weighted l - with the partials dealt to
+// more groups, so the order of the float64 additions differs.
+__device__ __forceinline__ double swap_sum(double x, int s) {
+  const uint64_t u = __double_as_longlong(x);
+  const float lo = __uint_as_float((uint32_t)u), hi = __uint_as_float((uint32_t)(u >> 32));
+  const uint32_t l = __float_as_uint(s == 32 ? lanes_xor<32>(lo) : lanes_xor<16>(lo));
+  const uint32_t h = __float_as_uint(s == 32 ? lanes_xor<32>(hi) : lanes_xor<16>(hi));
+  return x + __longlong_as_double((long long)((uint64_t)h << 32 | l));
+}
+template <int HD, int PARTS, int R>
 __global__ __launch_bounds__(kCombineThreads) void k_combine_part(DecodeParams P, float *q_out) {
   G2B_COMBINE_IN;
-  __shared__ float w[kCombineThreads];
-  __shared__ double gs[4 * kCombineThreads];  // [group][dims of the part]
-  __shared__ double red[kCombineThreads / 64];
-  const int h = (int)blockIdx.x / kCombineParts, part = (int)blockIdx.x - h * kCombineParts;
-  const int seq = blockIdx.y, li = blockIdx.z, tid = threadIdx.x;
-  const SeqDev sd = P.seqs ? P.seqs[seq] : P.one;
-  const int npos = sd.pos + 1;
-  const int np = (npos + P.split_len - 1) / P.split_len;
-  const int HD = P.sh.head_dim, nh = P.sh.n_heads, PD = HD / kCombineParts;
-  const size_t pstr = (size_t)(kPartHead + HD);
-  const size_t sidx = (size_t)li * (size_t)P.n_seq + (size_t)seq;
-  const float *base = P.part + (sidx * nh + h) * (size_t)P.max_splits * pstr;
-  const int tpr = PD / 4, GRP = kCombineThreads / tpr;  // (the host checks np <= GRP * R)
-  const int grp = tid / tpr, q = tid - grp * tpr;
-  // every load unconditional, as in k_combine's one-round path
-  float2 ml = *reinterpret_cast<const float2 *>(base + (size_t)min(tid, np - 1) * pstr);
-  if (tid >= np) ml = make_float2(kNegBig, 0.f);
-  float4 v[R];
-  const float *a = base + kPartHead + part * PD + 4 * q;
+  constexpr int PD = HD / PARTS, TPR = PD / 4, GRP = kCombineThreads / TPR;
+  constexpr int WG = TPR >= 64 ? 1 : (TPR >= 16 ? 1 : 16 / TPR);  // groups left per wave
+  constexpr int NW = kCombineThreads / 64, pstr = kPartHead + HD;
+  __shared__ float mx[NW];
+  __shared__ double gs[NW * WG * PD], gl[NW * WG];
+  const int h = (int)blockIdx.x / PARTS, part = (int)blockIdx.x - h * PARTS;
+  const int seq = blockIdx.y, li = blockIdx.z, tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const SeqDev *seqs = P.seqs;
+  const float *part_base = P.part;
+  float *const att = P.att;
+  const int n_seq = P.n_seq, nh = P.sh.n_heads, max_splits = P.max_splits, split_len = P.split_len;
+  int pos = P.one.pos;
+  asm volatile("" ::"s"(seqs), "s"(part_base), "s"(att), "s"(n_seq), "s"(nh), "s"(max_splits),
+               "s"(split_len), "s"(pos), "s"(q_out));
+  if (seqs) pos = *(const __attribute__((address_space(4))) int32_t *)(&seqs[seq].pos);
+  const int npos = pos + 1, np = (npos + split_len - 1) / split_len;
+  const size_t unit = (size_t)li * (size_t)n_seq + (size_t)seq;
+  const uint8_t *base = (const uint8_t *)(part_base + (unit * nh + h) * (size_t)max_splits * pstr);
+  const int grp = tid / TPR, q = tid - grp * TPR;
+  // (every load unconditional: a partial past np reads the last one and gets
+  // no weight)
+  typedef float f2 __attribute__((ext_vector_type(2)));
+  typedef float f4 __attribute__((ext_vector_type(4)));
+  f2 ml[R];
+  f4 v[R];
 #pragma unroll
   for (int u = 0; u < R; u++) {
-    const int p = min(grp + GRP * u, np - 1);
-    v[u] = *reinterpret_cast<const float4 *>(a + (size_t)p * pstr);
+    const uint32_t at = (uint32_t)min(grp + GRP * u, np - 1) * (pstr * 4u);
+    ml[u] = *(const __attribute__((address_space(1))) f2 *)(base + at);
+    v[u] = *(const __attribute__((address_space(1))) f4 *)(base + (at + 4u * (kPartHead + part * PD + 4 * q)));
   }
-  const float M = block_max_f(ml.x, reinterpret_cast<float *>(red));
-  double lsum = 0.0;
-  if (tid < np) {
-    const float wp = exp2f(ml.x - M);
-    w[tid] = wp;
-    lsum = (double)ml.y * (double)wp;
-  }
-  const double L = block_sum_d(lsum, red);  // (its barriers also publish w)
-  double o[4] = {0.0, 0.0, 0.0, 0.0};
+  float M = kNegBig;
+#pragma unroll
+  for (int u = 0; u < R; u++) M = fmaxf(M, ml[u].x);
+  M = fmaxf(M, dpp_f<0xB1>(M));
+  M = fmaxf(M, dpp_f<0x4E>(M));
+  M = fmaxf(M, dpp_f<0x141>(M));
+  M = fmaxf(M, dpp_f<0x140>(M));
+  M = fmaxf(M, lanes_xor<16>(M));
+  M = fmaxf(M, lanes_xor<32>(M));
+  if (lane == 0) mx[wave] = M;
+  barrier_lds();
+  M = fmaxf(fmaxf(mx[0], mx[1]), fmaxf(mx[2], mx[3]));
+  double o[4] = {0.0, 0.0, 0.0, 0.0}, l = 0.0;
 #pragma unroll
   for (int u = 0; u < R; u++) {
-    const int p = grp + GRP * u;
-    if (p < np) {
-      const double wp = (double)w[p];
-      o[0] = fma((double)v[u].x, wp, o[0]);
-      o[1] = fma((double)v[u].y, wp, o[1]);
-      o[2] = fma((double)v[u].z, wp, o[2]);
-      o[3] = fma((double)v[u].w, wp, o[3]);
+    const double wp = grp + GRP * u < np ? (double)exp2f(ml[u].x - M) : 0.0;
+    if (grp + GRP * u < np) {
+      l = fma((double)ml[u].y, wp, l);
+#pragma unroll
+      for (int j = 0; j < 4; j++) o[j] = fma((double)v[u][j], wp, o[j]);
     }
   }
-  for (int j = 0; j < 4; j++) gs[grp * PD + 4 * q + j] = o[j];
-  __syncthreads();
-  float *out = q_out + sidx * (size_t)(nh * HD) + (size_t)h * HD + (size_t)part * PD;
+  // the wave's groups that lie whole rows of 16 lanes apart
+  if constexpr (TPR <= 32) {
+    l = swap_sum(l, 32);
+#pragma unroll
+    for (int j = 0; j < 4; j++) o[j] = swap_sum(o[j], 32);
+  }
+  if constexpr (TPR <= 16) {
+    l = swap_sum(l, 16);
+#pragma unroll
+    for (int j = 0; j < 4; j++) o[j] = swap_sum(o[j], 16);
+  }
+  constexpr int KEEP = TPR >= 16 ? TPR : 16;  // lanes that hold the wave's sums
+  if (lane < KEEP) {
+    const int g = wave * WG + lane / TPR;
+#pragma unroll
+    for (int j = 0; j < 4; j++) gs[g * PD + 4 * q + j] = o[j];
+    if (q == 0) gl[g] = l;
+  }
+  barrier_lds();
+  float *out = q_out + unit * (size_t)(nh * HD) + (size_t)h * HD + (size_t)part * PD;
   for (int d = tid; d < PD; d += kCombineThreads) {
-    double sum = 0.0;
-    for (int g = 0; g < GRP; g++) sum += gs[g * PD + d];
+    double sum = 0.0, L = 0.0;
+#pragma unroll
+    for (int g = 0; g < NW * WG; g++) {
+      sum += gs[g * PD + d];
+      L += gl[g];
+    }
     out[d] = (float)(sum / L);
   }
-  if (P.att && part == 0) {
-    float *at = P.att + (sidx * nh + h) * (size_t)P.att_stride;
+  if (att && part == 0) {
+    double L = 0.0;
+#pragma unroll
+    for (int g = 0; g < NW * WG; g++) L += gl[g];
+    float *at = att + (unit * nh + h) * (size_t)P.att_stride;
     for (int t = tid; t < npos; t += blockDim.x)
       at[t] = (float)(exp2((double)at[t] - (double)M) / L);
   }
@@ -526,9 +570,42 @@ hipError_t launch_decode(const DecodeParams &p, int n_layers, hipStream_t s, boo
   return hipGetLastError();
 }
 
+// k_combine_part with the fewest rows per thread that cover the call's
+// partials (hipErrorInvalidValue: more than it holds).
+constexpr int64_t kCombinePartHeads = 1024;
+template <int HD, int PARTS, int R>
+static hipError_t launch_combine_r(const DecodeParams &p, int n_layers, hipStream_t s) {
+  const dim3 g((unsigned)(p.sh.n_heads * PARTS), (unsigned)p.n_seq, (unsigned)n_layers);
+  hipLaunchKernelGGL((k_combine_part<HD, PARTS, R>), g, dim3(kCombineThreads), 0, s, p, p.q_out);
+  return hipGetLastError();
+}
+template <int HD>
+static hipError_t launch_combine_part(const DecodeParams &p, int n_layers, hipStream_t s) {
+  constexpr int grp = kCombineThreads / (HD / 16);  // partials in one go, four parts
+  if ((int64_t)p.sh.n_heads * p.n_seq * n_layers > 256 && p.max_splits <= grp)
+    return launch_combine_r<HD, 1, 4>(p, n_layers, s);
+  if (p.max_splits <= grp) return launch_combine_r<HD, 4, 1>(p, n_layers, s);
+  if (p.max_splits <= 2 * grp) return launch_combine_r<HD, 4, 2>(p, n_layers, s);
+  if (p.max_splits <= 4 * grp) return launch_combine_r<HD, 4, 4>(p, n_layers, s);
+  if (p.max_splits <= 8 * grp) return launch_combine_r<HD, 4, 8>(p, n_layers, s);
+  return hipErrorInvalidValue;
+}
+
 hipError_t launch_combine(const DecodeParams &p, int n_layers, hipStream_t s) {
   if (p.max_splits > kCombineMaxParts) return hipErrorInvalidValue;
   dim3 grid(p.sh.n_heads, p.n_seq, n_layers);
+  // Static splits of few units: a workgroup per (head, quarter of its dims), so
+  // that one round of loads covers the partials and the heads reach more CUs;
+  // past 256 heads a workgroup per CU is there without the quarters.  Beyond
+  // kCombinePartHeads the launch is bound by starting workgroups (below).
+  const int hd = p.sh.head_dim;
+  const int64_t heads = (int64_t)p.sh.n_heads * p.n_seq * n_layers;
+  if (!p.wq && (hd == 64 || hd == 128 || hd == 256) && heads <= kCombinePartHeads) {
+    const hipError_t e = hd == 64    ? launch_combine_part<64>(p, n_layers, s)
+                         : hd == 128 ? launch_combine_part<128>(p, n_layers, s)
+                                     : launch_combine_part<256>(p, n_layers, s);
+    if (e != hipErrorInvalidValue) return e;
+  }
   // Few partials per head: one wave per head, four heads per workgroup.
   // With thousands of heads in the grid (c4: 4096) the launch is bound by
   // dispatching workgroups (~7 us to start 4096 of four waves), not by the
@@ -538,18 +615,6 @@ hipError_t launch_combine(const DecodeParams &p, int n_layers, hipStream_t s) {
     const int hpw = kCombineThreads / 64;  // heads per workgroup
     dim3 g4((p.sh.n_heads + hpw - 1) / hpw, p.n_seq, n_layers);
     hipLaunchKernelGGL(k_combine_waves, g4, dim3(kCombineThreads), 0, s, p, p.q_out);
-    return hipGetLastError();
-  }
-  // Static splits of few units with many partials: a workgroup per (head,
-  // quarter of its dims).
-  const int hd = p.sh.head_dim, grp = kCombineThreads / (hd / kCombineParts / 4);
-  if (!p.wq && hd % (4 * kCombineParts) == 0 && p.max_splits <= kCombineThreads &&
-      p.max_splits <= 8 * grp) {
-    dim3 gp(p.sh.n_heads * kCombineParts, p.n_seq, n_layers);
-    if (p.max_splits <= 4 * grp)
-      hipLaunchKernelGGL(k_combine_part<4>, gp, dim3(kCombineThreads), 0, s, p, p.q_out);
-    else
-      hipLaunchKernelGGL(k_combine_part<8>, gp, dim3(kCombineThreads), 0, s, p, p.q_out);
     return hipGetLastError();
   }
   hipLaunchKernelGGL(k_combine, grid, dim3(kCombineThreads), 0, s, p, p.q_out);

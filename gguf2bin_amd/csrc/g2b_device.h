@@ -54,6 +54,15 @@ __device__ __forceinline__ float wave_sum(float x) {
   return x + lanes_xor<32>(x);
 }
 
+// A workgroup barrier that orders LDS only: global loads issued before it stay
+// in flight across it (a full __syncthreads waits for every outstanding one),
+// and the compiler waits for each register where it is used.
+__device__ __forceinline__ void barrier_lds() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // Per-sequence descriptor as the kernels read it (32 bytes).
 struct SeqDev {
   int32_t pos;      // new token position; positions 0..pos are attended

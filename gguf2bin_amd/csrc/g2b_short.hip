@@ -220,17 +220,6 @@ __device__ __forceinline__ float wave_sum(float x) {
   return x;
 }
 
-// A workgroup barrier that orders LDS only: the phases up to the output
-// share nothing else, so the KV loads issued with the inputs stay in flight
-// through the norm, RoPE and append phases (a full __syncthreads waits for
-// every outstanding global load first); the compiler waits for each KV
-// register where the scores and V use it.
-__device__ __forceinline__ void barrier_lds() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 #ifdef G2B_STAMPS
 // Phase stamps of a k_short workgroup (thread 0; one-span calls): 0 entry,
 // 1 inputs and the norm factors in, 2 RoPE done, 3 append done, 4 scores
