@@ -336,12 +336,16 @@ def schedule_dict(shape: Shape, a) -> dict:
     instance they name for this shape (include/g2b_synth.h)."""
     kernel = KERNEL_NAMES.get(a[0], "none")
     wq = "true" if a[2] > 0 else "false"
-    if kernel == "k_layer":
+    group = shape.n_heads // shape.n_kv_heads
+    if a[7] == 1:
+        variant = (f"k_wide<{1 if shape.kv_q8 else 0}, {shape.head_dim}, "
+                   f"{1 if group <= 4 else 2 if group <= 8 else 4}>")
+    elif kernel == "k_layer":
         variant = (f"k_layer<{1 if shape.kv_q8 else 0}, {shape.head_dim}, {a[7]}, "
-                   f"{shape.n_heads // shape.n_kv_heads}, 2, {'true' if a[8] else 'false'}, "
+                   f"{group}, 2, {'true' if a[8] else 'false'}, "
                    f"{a[6]}, {wq}>")
     elif kernel == "k_tiles":
-        variant = f"k_tiles<{shape.n_heads // shape.n_kv_heads}, {wq}>"
+        variant = f"k_tiles<{group}, {wq}>"
     elif kernel == "k_short":
         variant = f"k_short<{1 if shape.kv_q8 else 0}, {shape.head_dim}>"
     else:
@@ -516,7 +520,8 @@ class Context:
         self._check(lib().g2b_ctx_tune(self.h, split_len, chunk, stage, piece), "g2b_ctx_tune")
 
     def tune_kernel(self, kernel: int):
-        """0 automatic, 1 k_layer only, 2 k_tiles where it applies, 3 spanned k_short."""
+        """0 automatic, 1 k_layer only, 2 k_tiles where it applies, 3 spanned k_short,
+        4 k_wide where it applies."""
         self._check(lib().g2b_ctx_tune_kernel(self.h, kernel), "g2b_ctx_tune_kernel")
 
     KERNEL_NAMES = KERNEL_NAMES

@@ -256,10 +256,55 @@ int32_t tiles_slots(g2b_ctx *c, bool wq) {
   return std::max(1, c->n_cu) * std::max(1, occ);
 }
 
-// Splits of k_wide that the device holds at once (cached).
+// Resident k_wide workgroups on the device (cached).
 int32_t wide_slots(g2b_ctx *c) {
   if (c->occ_wide <= 0) c->occ_wide = wide_blocks_per_cu(c->sh);
-  return std::max(1, c->n_cu * std::max(1, c->occ_wide) / wide_groups(c->sh));
+  return std::max(1, c->n_cu) * std::max(1, c->occ_wide);
+}
+
+// The positions a single unit (one sequence, one layer) is scheduled for: the
+// next power of two, so that a step at its own position and a captured step of
+// its bucket (g2b_model_use_graph: 64, 128, 256, ... positions) take the same
+// kernel and cut the context into the same splits.
+int64_t unit_positions(int32_t max_pos) {
+  int64_t n = 64;
+  while (n < (int64_t)max_pos + 1) n *= 2;
+  return n;
+}
+
+// Positions per k_wide split (one workgroup per KV head).  Up to kWideWhole
+// positions: the whole context, whose workgroups write the output (no combine;
+// 120 positions of one sequence, 8 KV heads, Q8_0: 9.2 us per layer in one
+// split, 10.3 in two and a combine).  Else at least one round of tiles, and so
+// long that the call's workgroups fit one round of the resident ones - one
+// past the round waits for another's setup and merge.  A single unit by whole
+// rounds of tiles: 8193 positions, 8 KV heads, Q8_0, 15.4 us per layer in 344
+// workgroups of 192 positions (16.0 in 520 of 128, 16.6 in 1032 of 64, 17.3 in
+// 264 of 256; 15.2 in 688 of 96, which 16383 positions would make 1368); 2049,
+// F32, 12.0 in 264 of 64 (11.4 in 208 of 80, 12.3 in 136 of 128, 13.9 in 88 of
+// 192).  A batch with half a split per sequence for the ragged ends and a tenth
+// to spare: 8 sequences of 1000-4000, 2 KV heads of 8 q heads, 16.6 us in 592
+// of 96 (19.4 in 896 of 64, 20.5 in 720 of 80, 17.2 in 448 of 128, 17.0 in 224
+// of 256).
+constexpr int32_t kWideWhole = 128;
+int32_t wide_split(const g2b_ctx *c, int64_t slots, int32_t n_seq, int64_t total_pos,
+                   int32_t max_pos, int32_t n_layers) {
+  const int64_t units = (int64_t)n_seq * n_layers, nkvh = c->shape.n_kv_heads;
+  int64_t sl;
+  if (max_pos < kWideWhole) {
+    sl = kWideWhole;
+  } else if (units == 1) {
+    const int64_t splits = std::max<int64_t>(slots / nkvh, 1);
+    sl = (unit_positions(max_pos) + splits * kWideRound - 1) / (splits * kWideRound) * kWideRound;
+  } else {
+    const int64_t splits = std::max<int64_t>(slots * 9 / 10 / nkvh - units / 2, 1);
+    sl = ((total_pos * n_layers + splits - 1) / splits + 15) / 16 * 16;
+  }
+  sl = std::max<int64_t>(sl, kWideRound);
+  if (c->split_override > 0) sl = c->split_override;
+  sl = std::max(sl, ((int64_t)max_pos + 512) / 512);
+  if (!decode_fast_available(c->sh)) sl = std::min<int64_t>(sl, kGenericMaxSplit);
+  return (int32_t)std::min<int64_t>(sl, (int64_t)max_pos + 1);
 }
 
 // Positions per split of a static schedule.  min_len is the shortest split
@@ -451,11 +496,13 @@ int run_layers(g2b_ctx *c, const SeqDev *d_seqs, const SeqDev &one, int32_t n_se
   // (k_layer reads q, k and v as 16-byte pieces; other pointers take the
   // generic kernels)
   const bool aligned = (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v) & 15u) == 0;
-  const bool fast = decode_fast_available(c->sh) && aligned;
-  // Shapes without a k_layer (wide GQA groups, many KV heads, head_dim 256):
-  // k_wide, one launch with the same partials.  Its splits keep the generic
-  // kernel's bounds (length, scratch), so a call that either refuses, both do.
-  const bool wide = !decode_fast_available(c->sh) && aligned && wide_available(c->sh);
+  const bool layer_shape = decode_fast_available(c->sh);
+  // k_wide: the shapes without a k_layer (wide GQA groups, many KV heads,
+  // head_dim 256), whose splits keep the generic kernel's bounds (length,
+  // scratch), so that a call that either refuses, both do; and the other shapes
+  // when a tuning asks for it.
+  const bool wide = aligned && wide_available(c->sh) && (!layer_shape || c->tune_kernel == 4);
+  const bool fast = layer_shape && aligned && !wide;
 
   DecodeParams dp{};
   dp.sh = c->sh;
@@ -506,7 +553,9 @@ int run_layers(g2b_ctx *c, const SeqDev *d_seqs, const SeqDev &one, int32_t n_se
   // the fixed scratch: k_short's span counters (kFixedCtrInts, kept zero),
   // the rotated q (generic path), then the partials
   const size_t fixed_ctr = fixed ? kFixedCtrInts : 0;
-  const size_t fixed_qrot = fixed && !fast ? ((size_t)n_layers * n_seq * nq + 63) & ~(size_t)63 : 0;
+  const size_t fixed_qrot = fixed && !fast && !(wide && layer_shape)
+                                ? ((size_t)n_layers * n_seq * nq + 63) & ~(size_t)63
+                                : 0;
   if (fixed) {
     const size_t per_split = (size_t)n_layers * n_seq * nh * (size_t)(kPartHead + hd);
     const size_t used = fixed_ctr + fixed_qrot;
@@ -664,9 +713,7 @@ int run_layers(g2b_ctx *c, const SeqDev *d_seqs, const SeqDev &one, int32_t n_se
     // (measured: four staged chunks or eight per-lane wave-steps per wave, four
     // for one layer of one sequence)
     const int32_t ppw = decode_ppw(c->sh, dp.tune_chunk);
-    // (k_wide: two tiles per wave; a split is wide_groups workgroups)
-    const int32_t min_len = wide                 ? 2 * wide_round(c->sh)
-                            : !fast              ? 64
+    const int32_t min_len = !fast                ? 64
                             : tiles             ? 8 * kTilesRows
                             : dp.stage_rows > 0 ? kWavesPerSplit * 4 * dp.stage_rows
                             : one_unit          ? kWavesPerSplit * 4 * ppw
@@ -698,8 +745,10 @@ int run_layers(g2b_ctx *c, const SeqDev *d_seqs, const SeqDev &one, int32_t n_se
                                 : one_unit   ? std::max(1, c->n_cu / 2)
                                 : n_seq == 1 ? std::max(1, c->n_cu)
                                              : slots * 7 / 10;
-    int32_t split_len = choose_split(c, std::max<int64_t>(split_slots, 1), n_seq, total_pos,
-                                     max_pos, n_layers, fast, min_len);
+    int32_t split_len =
+        wide ? wide_split(c, slots, n_seq, total_pos, max_pos, n_layers)
+             : choose_split(c, std::max<int64_t>(split_slots, 1), n_seq, total_pos, max_pos,
+                            n_layers, fast, min_len);
     if (fast && one_unit && dp.stage_rows == 0 && c->split_override == 0) {
       // whole trips (two wave-steps) for every wave: a wave with one more
       // trip than the others waits one more round trip (c1: 489 us per
@@ -707,15 +756,12 @@ int run_layers(g2b_ctx *c, const SeqDev *d_seqs, const SeqDev &one, int32_t n_se
       const int32_t trip = kWavesPerSplit * 2 * ppw;
       split_len = std::max(min_len, split_len / trip * trip);
     }
-    if (wide && c->split_override == 0)  // whole rounds of tiles
-      split_len = std::min<int32_t>(kGenericMaxSplit, (split_len + wide_round(c->sh) - 1) /
-                                                          wide_round(c->sh) * wide_round(c->sh));
     max_splits = (max_pos + 1 + split_len - 1) / split_len;
     if (max_splits > splits_per_seq) {  // lengthen the splits to stay within the budget
       split_len = (int32_t)(((int64_t)max_pos + splits_per_seq) / splits_per_seq);
       max_splits = (max_pos + 1 + split_len - 1) / split_len;
     }
-    if (!fast && split_len > kGenericMaxSplit)
+    if (!fast && !(wide && layer_shape) && split_len > kGenericMaxSplit)
       return fail(c, G2B_EUNSUP, "context %d of %d sequences needs splits of %d positions "
                   "(> %d on the generic kernel)", max_pos + 1, n_seq, split_len, kGenericMaxSplit);
     dp.split_len = split_len;
@@ -775,16 +821,22 @@ int run_layers(g2b_ctx *c, const SeqDev *d_seqs, const SeqDev &one, int32_t n_se
   // (what launch_layer instantiates: staging only with whole 16-byte row
   // pieces; k_tiles always pulls its tiles into LDS by DMA)
   const int32_t staging = tiles ? 1 : used_fast && dp.stage_rows > 0 ? dp.stage_mode : 0;
-  set_sched(c,
-            tiles       ? G2B_KERNEL_TILES
-            : wide      ? G2B_KERNEL_WIDE
-            : used_fast ? G2B_KERNEL_LAYER
-                        : G2B_KERNEL_GENERIC,
-            dp.split_len, use_wq ? dp.piece_len : 0, max_splits,
+  // (k_wide on k_layer's shapes: the kind of schedule - one split that writes
+  // the output, or splits and a combine; the chunk field says that k_wide ran)
+  const int32_t kernel = tiles                  ? G2B_KERNEL_TILES
+                         : wide ? !layer_shape  ? G2B_KERNEL_WIDE
+                                  : direct      ? G2B_KERNEL_SHORT
+                                                : G2B_KERNEL_LAYER
+                         : used_fast            ? G2B_KERNEL_LAYER
+                                                : G2B_KERNEL_GENERIC;
+  set_sched(c, kernel, dp.split_len, use_wq ? dp.piece_len : 0, max_splits,
             use_wq ? slots
-                   : (int64_t)max_splits * n_seq * n_layers * (wide ? wide_groups(c->sh) : 1),
-            direct && (used_fast || wide),
-            staging, used_fast && !tiles ? decode_chunk(c->sh, dp.tune_chunk) : 0, att != nullptr);
+                   : (int64_t)max_splits * n_seq * n_layers * (wide ? c->shape.n_kv_heads : 1),
+            direct && (used_fast || wide), staging,
+            wide                  ? 1
+            : used_fast && !tiles ? decode_chunk(c->sh, dp.tune_chunk)
+                                  : 0,
+            att != nullptr);
   if (ev1) G2B_HIP(c, hipEventRecord(ev1, c->stream));
   if (!direct || !(used_fast || wide)) G2B_HIP(c, launch_combine(dp, n_layers, c->stream));
   if (use_wq) {
@@ -1339,7 +1391,7 @@ int g2b_ctx_tune(g2b_ctx *c, int32_t split_len, int32_t chunk, int32_t stage, in
 }
 
 int g2b_ctx_tune_kernel(g2b_ctx *c, int32_t kernel) {
-  if (!c || kernel < 0 || kernel > 3) return G2B_EINVAL;
+  if (!c || kernel < 0 || kernel > 4) return G2B_EINVAL;
   c->tune_kernel = kernel;
   return G2B_OK;
 }

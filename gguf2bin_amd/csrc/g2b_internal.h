@@ -254,11 +254,10 @@ int tiles_blocks_per_cu(const ShapeDev &sh, bool wq);
 // as k_layer's.
 bool wide_available(const ShapeDev &sh);
 hipError_t launch_wide(const DecodeParams &p, int n_layers, hipStream_t s);
-// Its resident workgroups per CU, the KV-head groups (workgroups) of a split,
-// and the positions a workgroup's waves take per round of tiles.
+// Its resident workgroups per CU (a split is one per KV head), and the
+// positions a workgroup's four waves take per round of tiles.
 int wide_blocks_per_cu(const ShapeDev &sh);
-int wide_groups(const ShapeDev &sh);
-int wide_round(const ShapeDev &sh);
+constexpr int kWideRound = 64;
 template <int FMT, int HD>
 hipError_t launch_wide_hd(const DecodeParams &p, int n_layers, hipStream_t s);
 template <int FMT, int HD>

@@ -470,9 +470,6 @@ __device__ inline void append_new_row(const ShapeDev &sh, const SeqDev &sd, int 
 // they fit for every shape the specialised kernels take: n_heads * (hd/CD)
 // * (4 * CD/4 + 1) <= hd * (n_heads + n_kv_heads + 1) for CD 16 or 32 and
 // n_heads <= 4 * n_kv_heads.
-// slice_off, slice_bytes: sh may describe some of the KV heads of a row only
-// (n_heads, n_kv_heads; row_bytes stays the whole row's): the bytes they take
-// and where they start in it (0: the whole row).
 // The digit planes of a chunk: dig_stride<CD>() dwords (kQPlanes planes of
 // CD/4 dwords, 16-byte rows); the chunks' units 2^(e-30) follow all the
 // chunks' planes, one float each (dig_unit).
@@ -496,8 +493,7 @@ __device__ inline void visit_setup(const ShapeDev &sh, const SeqDev &sd, int lay
                                    const float *rope, const NormDev &norm, float qscale,
                                    float *qrot, float *kr, float *vr, uint8_t *rowk,
                                    uint8_t *rowv, float *scr, float *tr,
-                                   uint32_t *digp = nullptr, uint32_t slice_off = 0,
-                                   uint32_t slice_bytes = 0) {
+                                   uint32_t *digp = nullptr) {
   constexpr int half = HD / 2;
   constexpr int gph = half / 4;  // rope groups per head
   static_assert(half % 4 == 0, "four pairs per group");
@@ -705,13 +701,12 @@ __device__ inline void visit_setup(const ShapeDev &sh, const SeqDev &sd, int lay
   __syncthreads();
   if (!owns_new) return;
   const size_t off =
-      ((size_t)layer * (size_t)sd.ctx_cap + (size_t)sd.pos) * sh.row_bytes + slice_off;
-  const uint32_t store = slice_bytes ? slice_bytes : sh.row_bytes;
+      ((size_t)layer * (size_t)sd.ctx_cap + (size_t)sd.pos) * sh.row_bytes;
   uint32_t *gk = reinterpret_cast<uint32_t *>(sd.k + off);
   uint32_t *gv = reinterpret_cast<uint32_t *>(sd.v + off);
   const uint32_t *lk = reinterpret_cast<const uint32_t *>(rowk);
   const uint32_t *lv = reinterpret_cast<const uint32_t *>(rowv);
-  for (uint32_t i = threadIdx.x; i < store / 4; i += kThreads) {
+  for (uint32_t i = threadIdx.x; i < sh.row_bytes / 4; i += kThreads) {
     gk[i] = lk[i];
     gv[i] = lv[i];
   }

@@ -1,15 +1,17 @@
 // g2b_wide.hip - dispatch of k_wide (g2b_wide.h) over KV formats and head
 // sizes; the kernels are compiled by g2b_wide_inst.hip.
-#include "g2b_wide.h"
+#include "g2b_internal.h"
 
 namespace g2b {
 
-bool wide_available(const ShapeDev &sh) { return wide_shape_ok(sh); }
-int wide_groups(const ShapeDev &sh) { return sh.n_kv_heads / wide_kw(sh); }
-int wide_round(const ShapeDev &sh) { return kWideTile * (kWavesPerSplit / wide_kw(sh)); }
+bool wide_available(const ShapeDev &sh) {
+  if (sh.head_dim != 64 && sh.head_dim != 128 && sh.head_dim != 256) return false;
+  if (sh.n_kv_heads <= 0 || sh.n_heads % sh.n_kv_heads) return false;
+  return sh.n_heads / sh.n_kv_heads <= 16;
+}
 
 hipError_t launch_wide(const DecodeParams &p, int n_layers, hipStream_t s) {
-  if (!wide_shape_ok(p.sh)) return hipErrorInvalidValue;
+  if (!wide_available(p.sh)) return hipErrorInvalidValue;
   if (p.sh.kv_q8) {
     switch (p.sh.head_dim) {
       case 64: return launch_wide_hd<1, 64>(p, n_layers, s);
@@ -25,7 +27,7 @@ hipError_t launch_wide(const DecodeParams &p, int n_layers, hipStream_t s) {
 }
 
 int wide_blocks_per_cu(const ShapeDev &sh) {
-  if (!wide_shape_ok(sh)) return 1;
+  if (!wide_available(sh)) return 1;
   if (sh.kv_q8) {
     switch (sh.head_dim) {
       case 64: return wide_occupancy_hd<1, 64>(sh);
