@@ -668,6 +668,8 @@ def phases_leg(w: Workload, steps: int, warmup: int) -> dict:
     ctx, s = w.ctx, w.shape
     khz = hip.wall_clock_khz(0)
     cap = max(4096, w.n_seq * 64)
+    if w.n_seq == 1:
+        ctx.tune_kernel(1)  # (only k_layer stamps; the automatic choice is k_wide)
     ctx.stamps_enable(cap, s.n_layers)
     for _ in range(max(1, warmup)):
         w.step_layer_serial()

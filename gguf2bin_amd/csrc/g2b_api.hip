@@ -307,6 +307,42 @@ int32_t wide_split(const g2b_ctx *c, int64_t slots, int32_t n_seq, int64_t total
   return (int32_t)std::min<int64_t>(sl, (int64_t)max_pos + 1);
 }
 
+// Calls on k_layer's shapes that k_wide serves: those bound by latency, where
+// one KV head per workgroup and a setup that runs while the first tiles come
+// are shorter than k_short's and k_layer's chains, which cover all heads.  us
+// per layer, layer-serial, before -> k_wide (16 / 8 heads of 128 unless said):
+//  - below kWideWhole positions, any batch (k_short): Q8_0 at 47 positions 8.6
+//    -> 5.9, 126 positions 11.4 -> 8.7; 64 sequences of 50-103 14.7 -> 12.3, 256
+//    of them 35.8 -> 29.6 (9 / 3 of 64 14.6 -> 11.9); F32 rows of 4 KB 256 of
+//    50-103 (163 MB) 48.1 -> 47.3, but 256 of 64-127 (200 MB) 51.4 -> 52.3;
+//  - one layer of one sequence (k_layer; 32 / 8 of 128, Q8_0: k_tiles): Q8_0 at
+//    1000 13.9 -> 9.0, 8192 16.9 -> 15.5, 32767 33.3 -> 30.8; F32 at 2048 13.2 ->
+//    12.1, 32767 73 -> 54, but 8192 24.4 -> 26.4, 9000 24.7 -> 27.0 (splits cut
+//    for 16384 positions leave CUs idle; 11000 29.6 -> 28.1); 32 / 8, Q8_0 at
+//    1000 25.5 -> 9.1, 16383 28.6 -> 20.8, but 32767 30.2 -> 31.0;
+//  - up to 64 units of at most 512 positions: 8 sequences of 150-303, Q8_0 20.2
+//    -> 11.4, 32 of 255-511 51.6 -> 20.6, 64 56.7 -> 43.8; F32 16 of 150-303 (30
+//    MB) 20.1 -> 16.3, but 32 of 255-511 29.4 -> 30.7;
+//  - few KV bytes in all: 2 sequences of 500-1003 (3.3 MB, Q8_0) 19.8 -> 10.7, 8
+//    of 550-1103 (14 MB) 20.2 -> 18.2, 2 of 650-1299 (16 MB, F32) 16.4 -> 12.4,
+//    8 of 3250-6499, 9 / 3 of 64 (16 MB, Q8_0) 18.8 -> 15.6; past that k_layer's
+//    longer streams win (4 of 1500-3003, F32, 74 MB 24.0 -> 25.5; 64 of 750-1503,
+//    9 / 3, Q8_0, 29 MB 23.4 -> 25.5).  k_tiles has the longest setup: 16 of
+//    1000-2003, 32 / 8, Q8_0 (52 MB) 34.5 -> 29.0, 32 of 500-999 (52 MB) 68.8 ->
+//    29.5, 64 of 750-1503 (157 MB) 70.5 -> 101.6.
+bool wide_latency(const ShapeDev &sh, int32_t n_seq, int32_t n_layers, int32_t max_pos,
+                  int64_t total_pos) {
+  constexpr int64_t kMB = 1 << 20;
+  const int64_t units = (int64_t)n_seq * n_layers;
+  const int64_t bytes = total_pos * n_layers * 2 * (int64_t)sh.row_bytes;
+  const bool t = tiles_available(sh), f32_4k = !sh.kv_q8 && sh.row_bytes >= 4096;
+  if (max_pos < kWideWhole) return !f32_4k || bytes <= 160 * kMB;
+  if (units == 1)
+    return t ? unit_positions(max_pos) <= 16384 : !(f32_4k && max_pos >= 8192 && max_pos < 10240);
+  if (units <= 64 && max_pos < 512) return !f32_4k || bytes <= 32 * kMB;
+  return bytes <= (t ? 52 : 16) * kMB;
+}
+
 // Positions per split of a static schedule.  min_len is the shortest split
 // worth a workgroup (its waves get a few wave-steps or chunks each; shorter
 // splits cost more in setup and partials than they gain).
@@ -500,8 +536,13 @@ int run_layers(g2b_ctx *c, const SeqDev *d_seqs, const SeqDev &one, int32_t n_se
   // k_wide: the shapes without a k_layer (wide GQA groups, many KV heads,
   // head_dim 256), whose splits keep the generic kernel's bounds (length,
   // scratch), so that a call that either refuses, both do; and the other shapes
-  // when a tuning asks for it.
-  const bool wide = aligned && wide_available(c->sh) && (!layer_shape || c->tune_kernel == 4);
+  // where wide_latency says so or a tuning asks for it.
+  const bool untuned = c->tune_kernel == 0 && c->split_override == 0 && c->tune_piece == 0 &&
+                       c->tune_chunk == 0 && c->tune_stage == 0;
+  const bool wide =
+      aligned && wide_available(c->sh) &&
+      (!layer_shape || c->tune_kernel == 4 ||
+       (untuned && !att && wide_latency(c->sh, n_seq, n_layers, max_pos, total_pos)));
   const bool fast = layer_shape && aligned && !wide;
 
   DecodeParams dp{};
@@ -566,8 +607,8 @@ int run_layers(g2b_ctx *c, const SeqDev *d_seqs, const SeqDev &one, int32_t n_se
     splits_per_seq = (int32_t)std::min<size_t>((size_t)splits_per_seq, fit);
   }
 
-  // k_short, no weights output: one workgroup per (KV head, span of
-  // kShortMaxPos positions, sequence, layer).  Below kShortMaxPos positions
+  // k_short, no weights output, where k_wide is not taken (a tuning, or F32
+  // rows of 4 KB in large batches): one workgroup per (KV head, span of kShortMaxPos positions, sequence, layer).  Below kShortMaxPos positions
   // it is a single span that writes the output over q itself.  Longer
   // contexts take it (spans that merge their partials in the kernel, no
   // combine launch) only when g2b_ctx_tune_kernel(3) asks for it: one layer

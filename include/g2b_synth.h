@@ -58,14 +58,16 @@ int g2b_synth_copy(g2b_ctx *ctx, void *dst, const void *src, uint64_t nbytes);
 int g2b_ctx_tune(g2b_ctx *ctx, int32_t split_len, int32_t chunk, int32_t stage, int32_t piece);
 
 /* Decode kernel choice.  0 automatic: k_wide (one KV head per workgroup) for
- * shapes without a k_layer; k_tiles (K scores on the int8 matrix cores) for
- * Q8_0 KV with head_dim 128, 8 KV heads and 3-4 q heads per KV head when
- * neither the weights output, a chunk nor a stage other than 2 is asked for;
- * else k_layer.  1: k_layer (no k_tiles, no spans).  2: k_tiles where it
- * applies, no spans.  3: spans of k_short wherever they apply (any batch), else
- * k_tiles or k_layer.  4: k_wide wherever it applies.  In modes 0 to 3 contexts
- * below 128 positions take the single-span k_short unless g2b_ctx_tune sets a
- * split length or piece. */
+ * shapes without a k_layer, and, without the weights output and without a
+ * g2b_ctx_tune, for the calls of the others that latency bounds (contexts
+ * below 128 positions, one layer of one sequence, few KV bytes in all);
+ * k_tiles (K scores on the int8 matrix cores) for Q8_0 KV with head_dim 128,
+ * 8 KV heads and 3-4 q heads per KV head when neither the weights output, a
+ * chunk nor a stage other than 2 is asked for; else k_layer.  1: k_layer (no
+ * k_tiles, no spans).  2: k_tiles where it applies, no spans.  3: spans of
+ * k_short wherever they apply (any batch), else k_tiles or k_layer.  4: k_wide
+ * wherever it applies.  In modes 1 to 3 contexts below 128 positions take the
+ * single-span k_short unless g2b_ctx_tune sets a split length or piece. */
 int g2b_ctx_tune_kernel(g2b_ctx *ctx, int32_t kernel);
 
 /* The schedule of the last decode call that launched (g2b_attn_layers,

@@ -1,0 +1,43 @@
+"""Which calls of k_layer's shapes the automatic choice gives to k_wide, on
+both sides of each line of the rule, against the oracle."""
+from __future__ import annotations
+
+import pytest
+
+from oracle import orc
+from test_gpu_parity import run_batch_case
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = {
+    "qwen3_q8": (16, 8, 128, orc.ARCH_QWEN3, True),
+    "qwen3_f32": (16, 8, 128, orc.ARCH_QWEN3, False),
+    "smollm2_q8": (9, 3, 64, orc.ARCH_LLAMA, True),
+    "llama3_q8": (32, 8, 128, orc.ARCH_LLAMA, True),
+}
+CASES = [
+    ("qwen3_q8", [127], False, "k_wide"),
+    ("qwen3_q8", [700], False, "k_wide"),
+    ("qwen3_q8", [700], True, "k_layer"),  # the weights output
+    ("smollm2_q8", [0, 127, 64], False, "k_wide"),
+    ("smollm2_q8", [511, 128, 4], False, "k_wide"),
+    # 2 x 4096 bytes a position: 2048 positions are the 16 MiB of a batch
+    ("qwen3_f32", [1023, 1023], False, "k_wide"),
+    ("qwen3_f32", [1024, 1023], False, "k_layer"),
+    ("qwen3_f32", [8191], False, "k_wide"),
+    ("qwen3_f32", [8192], False, "k_layer"),
+    ("llama3_q8", [16383], False, "k_wide"),
+    ("llama3_q8", [16384], False, "k_tiles"),
+]
+
+
+@pytest.mark.parametrize("name,poss,att,kernel", CASES, ids=str)
+def test_choice(gpu_device, name, poss, att, kernel):
+    nh, nkv, hd, arch, q8 = SHAPES[name]
+    o = orc.Shape(1, nh, nkv, hd, 1e5, arch, q8)
+    # (rows of 204 bytes: whole capacities of eight rows keep caches aligned)
+    caps = [(p // 8 + 1) * 8 for p in poss]
+    print(f"[choice] {name} {poss} att={att}", flush=True)
+    sched = {}
+    run_batch_case(o, caps, poss, seed=71, fused=False, want_att=att, sched=sched)
+    assert sched["variant"].startswith(kernel + "<"), sched
