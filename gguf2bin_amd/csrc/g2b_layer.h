@@ -291,7 +291,7 @@ constexpr int kQBits = 8 * kQPlanes - 2;  // 30
 template <int CD>
 struct QDigits {
   uint32_t d[kQPlanes][CD / 4];
-  float unit;  // 2^(e-30): value of one m step
+  float unit;  // 2^(e-30): value of one m step (NaN: a non-finite q, digit_scale)
 };
 
 // The digits of m (|m| <= 2^30): planes 0..2 in [-128, 127], plane 3 the
@@ -305,16 +305,29 @@ __device__ __forceinline__ void split_digits(int m, int (&d)[kQPlanes]) {
   d[kQPlanes - 1] = m;
 }
 
+// 2^(kQBits-e) and 2^(e-kQBits) of a chunk whose largest |q| has the bits mx
+// (abs_bits).  A chunk that holds an Inf or a NaN has no digits: they are 0
+// and the unit is NaN, so every score of its head, and with them the head's
+// output, is NaN, as in the fp32 dot (Inf in q meets both signs of k; the
+// softmax of infinite scores is NaN).
+struct DigitScale {
+  float up, unit;
+};
+__device__ __forceinline__ DigitScale digit_scale(uint32_t mx) {
+  int e = 0;
+  (void)frexpf(__uint_as_float(mx), &e);
+  if (mx >= kInfBits) return {0.f, __int_as_float(0x7fc00000)};
+  return {ldexpf(1.f, kQBits - e), ldexpf(1.f, e - kQBits)};
+}
+
 template <int CD>
 __device__ __forceinline__ QDigits<CD> make_digits(const float (&q)[CD]) {
   QDigits<CD> r;
-  float mx = 0.f;
+  uint32_t mx = 0u;
 #pragma unroll
-  for (int j = 0; j < CD; j++) mx = fmaxf(mx, fabsf(q[j]));
-  int e = 0;
-  (void)frexpf(mx, &e);
-  const float up = ldexpf(1.f, kQBits - e);
-  r.unit = ldexpf(1.f, e - kQBits);
+  for (int j = 0; j < CD; j++) mx = max(mx, abs_bits(q[j]));
+  const DigitScale ds = digit_scale(mx);
+  r.unit = ds.unit;
 #pragma unroll
   for (int k = 0; k < kQPlanes; k++)
 #pragma unroll
@@ -322,7 +335,7 @@ __device__ __forceinline__ QDigits<CD> make_digits(const float (&q)[CD]) {
 #pragma unroll
   for (int j = 0; j < CD; j++) {
     int d[kQPlanes];
-    split_digits((int)rintf(q[j] * up), d);
+    split_digits((int)rintf(q[j] * ds.up), d);
     const int sh = 8 * (j & 3);
 #pragma unroll
     for (int k = 0; k < kQPlanes; k++) r.d[k][j >> 2] |= ((uint32_t)d[k] & 0xffu) << sh;
@@ -648,14 +661,12 @@ __device__ inline void visit_setup(const ShapeDev &sh, const SeqDev &sd, int lay
         q[j + 2] = v4.z * qscale;
         q[j + 3] = v4.w * qscale;
       }
-      float mx = 0.f;
+      uint32_t mx = 0u;
 #pragma unroll
-      for (int j = 0; j < QE; j++) mx = fmaxf(mx, fabsf(q[j]));
-      mx = fmaxf(mx, __shfl_xor(mx, 1));
-      mx = fmaxf(mx, __shfl_xor(mx, 2));
-      int e = 0;
-      (void)frexpf(mx, &e);
-      const float up = ldexpf(1.f, kQBits - e);
+      for (int j = 0; j < QE; j++) mx = max(mx, abs_bits(q[j]));
+      mx = max(mx, (uint32_t)__shfl_xor((int)mx, 1));
+      mx = max(mx, (uint32_t)__shfl_xor((int)mx, 2));
+      const DigitScale ds = digit_scale(mx);
       uint32_t d[kQPlanes][QE / 4];
 #pragma unroll
       for (int pl = 0; pl < kQPlanes; pl++)
@@ -664,7 +675,7 @@ __device__ inline void visit_setup(const ShapeDev &sh, const SeqDev &sd, int lay
 #pragma unroll
       for (int j = 0; j < QE; j++) {
         int dj[kQPlanes];
-        split_digits((int)rintf(q[j] * up), dj);
+        split_digits((int)rintf(q[j] * ds.up), dj);
         const int sh8 = 8 * (j & 3);
 #pragma unroll
         for (int pl = 0; pl < kQPlanes; pl++) d[pl][j >> 2] |= ((uint32_t)dj[pl] & 0xffu) << sh8;
@@ -674,7 +685,7 @@ __device__ inline void visit_setup(const ShapeDev &sh, const SeqDev &sd, int lay
       for (int pl = 0; pl < kQPlanes; pl++)
 #pragma unroll
         for (int j = 0; j < QE / 4; j++) o[pl * (CD / 4) + k * (QE / 4) + j] = d[pl][j];
-      if (k == 0) dig[dig_unit_at<CD>(nch, ch)] = __float_as_uint(ldexpf(1.f, e - kQBits));
+      if (k == 0) dig[dig_unit_at<CD>(nch, ch)] = __float_as_uint(ds.unit);
     }
   }
   if (owns_new) {

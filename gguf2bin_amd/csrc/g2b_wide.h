@@ -349,26 +349,28 @@ __global__ __launch_bounds__(kThreads) void k_wide(DecodeParams P, int z0) {
     } else {
       // make_digits' digits: a block's largest |q| over its lanes (eight of
       // a, eight of b; LLaMA: four of both)
-      float ma = fmaxf(fmaxf(fabsf(a[0]), fabsf(a[1])), fmaxf(fabsf(a[2]), fabsf(a[3])));
-      float mb = fmaxf(fmaxf(fabsf(b[0]), fabsf(b[1])), fmaxf(fabsf(b[2]), fabsf(b[3])));
-      if (llama) ma = mb = fmaxf(ma, mb);
-      ma = fmaxf(ma, dpp_f<0xB1>(ma));
-      mb = fmaxf(mb, dpp_f<0xB1>(mb));
-      ma = fmaxf(ma, dpp_f<0x4E>(ma));
-      mb = fmaxf(mb, dpp_f<0x4E>(mb));
-      if (!llama) {
-        ma = fmaxf(ma, dpp_f<0x141>(ma));
-        mb = fmaxf(mb, dpp_f<0x141>(mb));
+      uint32_t ma = 0u, mb = 0u;
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        ma = max(ma, abs_bits(a[j]));
+        mb = max(mb, abs_bits(b[j]));
       }
-      auto put = [&](const f32x4 &x, float mx, int e) {
-        int ex = 0;
-        (void)frexpf(mx, &ex);
-        const float up = ldexpf(1.f, kQBits - ex);
+      if (llama) ma = mb = max(ma, mb);
+      ma = max(ma, dpp_u<0xB1>(ma));
+      mb = max(mb, dpp_u<0xB1>(mb));
+      ma = max(ma, dpp_u<0x4E>(ma));
+      mb = max(mb, dpp_u<0x4E>(mb));
+      if (!llama) {
+        ma = max(ma, dpp_u<0x141>(ma));
+        mb = max(mb, dpp_u<0x141>(mb));
+      }
+      auto put = [&](const f32x4 &x, uint32_t mx, int e) {
+        const DigitScale ds = digit_scale(mx);
         uint32_t d[kQPlanes] = {0u, 0u, 0u, 0u};
 #pragma unroll
         for (int j = 0; j < 4; j++) {
           int dj[kQPlanes];
-          split_digits((int)rintf(x[j] * up), dj);
+          split_digits((int)rintf(x[j] * ds.up), dj);
 #pragma unroll
           for (int p = 0; p < kQPlanes; p++) d[p] |= ((uint32_t)dj[p] & 0xffu) << (8 * j);
         }
@@ -378,7 +380,7 @@ __global__ __launch_bounds__(kThreads) void k_wide(DecodeParams P, int z0) {
 #pragma unroll
           for (int p = 0; p < kQPlanes; p++) o[p * 8] = d[p];
           if ((e & 31) == 0)
-            digs[dig_unit_at<32>(NCH, ch)] = __float_as_uint(ldexpf(1.f, ex - kQBits));
+            digs[dig_unit_at<32>(NCH, ch)] = __float_as_uint(ds.unit);
         }
       };
       put(a, ma, oa);
