@@ -272,6 +272,15 @@ __device__ __forceinline__ void lane_x(const GemvParams &P, const float *xs, int
   }
 }
 
+// The largest |x| of a block, as bits (abs_bits: Inf and NaN lie at and above
+// kInfBits), from the four elements that each of its eight lanes holds.
+__device__ __forceinline__ uint32_t block_abs_bits(const float4 &v) {
+  uint32_t mx = max(max(abs_bits(v.x), abs_bits(v.y)), max(abs_bits(v.z), abs_bits(v.w)));
+#pragma unroll
+  for (int o = 1; o < 8; o *= 2) mx = max(mx, (uint32_t)__shfl_xor((int)mx, o));
+  return mx;
+}
+
 // x as four signed int8 digit planes of a 31-bit fixed point per 32-element
 // block (the Q8_0 XD form): m = rint(x * 2^(30-e)), 2^(e-1) <= max|x| < 2^e,
 // m = d0 + 256 d1 + 65536 d2 + 2^24 d3.  The workgroup makes every block's
@@ -292,12 +301,9 @@ __device__ __forceinline__ void wg_x_digits(const GemvParams &P, const float *xs
     const int b = it >> 3, j = it & 7;  // chunk j: elements 4j .. 4j+3 of block b
     const float4 v = P.pro == kProNone ? reinterpret_cast<const float4 *>(P.x)[it]
                                        : staged_x4(P, xs, b, j, inv);
-    float mx = fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)));
-    mx = fmaxf(mx, __shfl_xor(mx, 1));
-    mx = fmaxf(mx, __shfl_xor(mx, 2));
-    mx = fmaxf(mx, __shfl_xor(mx, 4));
+    const uint32_t mx = block_abs_bits(v);
     int e = 0;
-    (void)frexpf(mx, &e);
+    (void)frexpf(__uint_as_float(mx), &e);
     const float xv[4] = {v.x, v.y, v.z, v.w};
     uint32_t pl[4] = {0u, 0u, 0u, 0u};
 #pragma unroll
@@ -317,7 +323,7 @@ __device__ __forceinline__ void wg_x_digits(const GemvParams &P, const float *xs
     for (int q = 0; q < 4; q++) dig[(b * 4 + q) * 8 + j] = pl[q];
     if (j == 0) {
       exps[b] = e;
-      units[b] = (mx <= 3.402823466e38f) ? 1.f : __int_as_float(0x7fc00000);
+      units[b] = mx < kInfBits ? 1.f : __int_as_float(0x7fc00000);
     }
   }
   __syncthreads();
@@ -663,12 +669,9 @@ __global__ __launch_bounds__(kGemvThreads) void k_gemv_mma(GemvParams P) {
     for (int it = threadIdx.x; it < NB * 8; it += kGemvThreads) {
       const int b = it >> 3, j = it & 7;  // chunk j: elements 4j .. 4j+3
       const float4 v = *reinterpret_cast<const float4 *>(P.x + 32 * b + 4 * j);
-      float mx = fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)));
-      mx = fmaxf(mx, __shfl_xor(mx, 1));
-      mx = fmaxf(mx, __shfl_xor(mx, 2));
-      mx = fmaxf(mx, __shfl_xor(mx, 4));
+      const uint32_t mx = block_abs_bits(v);
       int e = 0;
-      (void)frexpf(mx, &e);
+      (void)frexpf(__uint_as_float(mx), &e);
       const float xv[4] = {v.x, v.y, v.z, v.w};
       uint32_t pl[4] = {0u, 0u, 0u, 0u};
       int ps[4] = {0, 0, 0, 0};
@@ -701,7 +704,7 @@ __global__ __launch_bounds__(kGemvThreads) void k_gemv_mma(GemvParams P) {
         // the block's exponent, and 1 (NaN for a non-finite x: the rows'
         // sums then are NaN)
         exps[b] = e;
-        units[b] = (mx <= 3.402823466e38f) ? 1.f : __int_as_float(0x7fc00000);
+        units[b] = mx < kInfBits ? 1.f : __int_as_float(0x7fc00000);
 #pragma unroll
         for (int q = 0; q < 4; q++) dsum[b * 4 + q] = ps[q];
       }
