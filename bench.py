@@ -577,10 +577,18 @@ def model_leg(args):
             for i in range(8, 8 + K):
                 m.forward(toks[i], i)
             dt = (time.perf_counter() - t0) / K
+            mctx = attn.lib().g2b_model_ctx(m.h)
+
+            def schedule():
+                sched = (C.c_int32 * attn.SCHED_FIELDS)()
+                attn.lib().g2b_ctx_last_schedule(mctx, sched)
+                return attn.schedule_dict(attn.Shape(cfg["n_layers"], 16, 8, 128, 1e6,
+                                                     attn.ARCH_QWEN3, True), sched)
+
+            ssched = schedule()
             # the long window: positions 0..P0-1 of every layer filled on the
             # device (seeded N(0,1) rows through the append arithmetic)
             kc, vc, cap = m.kv()
-            mctx = attn.lib().g2b_model_ctx(m.h)
             rc = attn.lib().g2b_synth_fill_kv(mctx, kc, vc, cap, 0, cfg["n_layers"], 0, P0,
                                               args.seed, 0, float("inf"))
             if rc or attn.lib().g2b_sync(mctx):
@@ -595,27 +603,23 @@ def model_leg(args):
             for i in range(4, 4 + K):
                 m.forward(ltoks[i], P0 + i)
             ldt = (time.perf_counter() - t0) / K
-            sched = (C.c_int32 * attn.SCHED_FIELDS)()
-            attn.lib().g2b_ctx_last_schedule(mctx, sched)
-            lsched = attn.schedule_dict(attn.Shape(cfg["n_layers"], 16, 8, 128, 1e6,
-                                                   attn.ARCH_QWEN3, True), sched)
+            lsched = schedule()
             kv_cap = cap
         res = {"workload": "Qwen3-0.6B shape, random Q8_0 weights (tied embeddings, QK-RMSNorm), "
                            "Q8_0 KV, batch 1",
                "weight_bytes": int(wbytes),
                "short_context": {
-                   "positions": f"8..{8 + K - 1}", "attention": "k_short, one span",
+                   "positions": f"8..{8 + K - 1}", "attention_schedule": ssched,
                    "ms_per_token": round(dt * 1e3, 3), "tokens_per_s": round(1 / dt, 1),
                    "weight_GBps": round(wbytes / dt / 1e9, 1),
-                   # embedding, 5 per layer (four fused GEMVs and the attention),
-                   # logits
-                   "launches_per_token": cfg["n_layers"] * 5 + 2},
+                   # embedding, per layer four fused GEMVs and the attention (and
+                   # its combine, where it has several splits), logits
+                   "launches_per_token": cfg["n_layers"] * (
+                       5 if ssched["output_in_kernel"] else 6) + 2},
                "long_context": {
                    "positions": f"{P0}..{P0 + 3 + K}", "kv_positions_filled": P0,
                    "attention_schedule": lsched,
                    "ms_per_token": round(ldt * 1e3, 3), "tokens_per_s": round(1 / ldt, 1),
-                   # plus the combine launch per layer where the splits are not
-                   # merged in the decode kernel
                    "launches_per_token": cfg["n_layers"] * (
                        5 if lsched["output_in_kernel"] else 6) + 2}}
         if have_ref:

@@ -337,7 +337,7 @@ def schedule_dict(shape: Shape, a) -> dict:
     kernel = KERNEL_NAMES.get(a[0], "none")
     wq = "true" if a[2] > 0 else "false"
     group = shape.n_heads // shape.n_kv_heads
-    if a[7] == 1:
+    if kernel == "k_wide":
         variant = (f"k_wide<{1 if shape.kv_q8 else 0}, {shape.head_dim}, "
                    f"{1 if group <= 4 else 2 if group <= 8 else 4}>")
     elif kernel == "k_layer":

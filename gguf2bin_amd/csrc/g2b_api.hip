@@ -862,22 +862,15 @@ int run_layers(g2b_ctx *c, const SeqDev *d_seqs, const SeqDev &one, int32_t n_se
   // (what launch_layer instantiates: staging only with whole 16-byte row
   // pieces; k_tiles always pulls its tiles into LDS by DMA)
   const int32_t staging = tiles ? 1 : used_fast && dp.stage_rows > 0 ? dp.stage_mode : 0;
-  // (k_wide on k_layer's shapes: the kind of schedule - one split that writes
-  // the output, or splits and a combine; the chunk field says that k_wide ran)
-  const int32_t kernel = tiles                  ? G2B_KERNEL_TILES
-                         : wide ? !layer_shape  ? G2B_KERNEL_WIDE
-                                  : direct      ? G2B_KERNEL_SHORT
-                                                : G2B_KERNEL_LAYER
-                         : used_fast            ? G2B_KERNEL_LAYER
-                                                : G2B_KERNEL_GENERIC;
+  const int32_t kernel = tiles       ? G2B_KERNEL_TILES
+                         : wide      ? G2B_KERNEL_WIDE
+                         : used_fast ? G2B_KERNEL_LAYER
+                                     : G2B_KERNEL_GENERIC;
   set_sched(c, kernel, dp.split_len, use_wq ? dp.piece_len : 0, max_splits,
             use_wq ? slots
                    : (int64_t)max_splits * n_seq * n_layers * (wide ? c->shape.n_kv_heads : 1),
             direct && (used_fast || wide), staging,
-            wide                  ? 1
-            : used_fast && !tiles ? decode_chunk(c->sh, dp.tune_chunk)
-                                  : 0,
-            att != nullptr);
+            used_fast && !tiles ? decode_chunk(c->sh, dp.tune_chunk) : 0, att != nullptr);
   if (ev1) G2B_HIP(c, hipEventRecord(ev1, c->stream));
   if (!direct || !(used_fast || wide)) G2B_HIP(c, launch_combine(dp, n_layers, c->stream));
   if (use_wq) {

@@ -72,10 +72,7 @@ int g2b_ctx_tune_kernel(g2b_ctx *ctx, int32_t kernel);
 
 /* The schedule of the last decode call that launched (g2b_attn_layers,
  * g2b_attn_forward and their variants), into out[G2B_SCHED_FIELDS]:
- *   [0] schedule: G2B_KERNEL_LAYER (splits and a combine, or the work queue),
- *       _TILES, _SHORT (one split that writes the output, or spans), _GENERIC,
- *       or _WIDE (shapes without a k_layer); a k_layer shape that ran on k_wide
- *       is _LAYER or _SHORT with [7] = 1,
+ *   [0] kernel: G2B_KERNEL_LAYER, _TILES, _SHORT, _GENERIC or _WIDE,
  *   [1] positions per split (k_short: per span; 0 under the work queue),
  *   [2] work-queue piece length (0: static splits or spans),
  *   [3] partial slots per (sequence, layer) (splits, spans or queue slots),
@@ -85,13 +82,12 @@ int g2b_ctx_tune_kernel(g2b_ctx *ctx, int32_t kernel);
  *   [6] how KV rows reach the lanes: 0 per-lane loads straight from HBM,
  *       1 chunks (k_tiles: tiles) pulled into LDS by LDS DMA, 2 chunks
  *       loaded into registers one chunk ahead and written to LDS,
- *   [7] k_layer: row elements per lane (32 = a Q8_0 block, 16); 1 when the
- *       kernel is k_wide (one KV head per workgroup), whatever [0]; else 0,
+ *   [7] k_layer: row elements per lane (32 = a Q8_0 block, 16); else 0,
  *   [8] 1 when the call wrote the softmax weights.
  * With the shape, [0], [2], [6], [7] and [8] name the kernel instance
  * launched: k_layer<kv_q8, head_dim, [7], group, 2, [8], [6], [2] > 0>,
- * k_tiles<group, [2] > 0>, or with [7] = 1 k_wide<kv_q8, head_dim, sets of
- * four q heads per KV head: 1, 2 or 4>.  All zero before the first call. */
+ * k_tiles<group, [2] > 0>, or k_wide<kv_q8, head_dim, sets of four q heads
+ * per KV head: 1, 2 or 4>.  All zero before the first call. */
 #define G2B_SCHED_FIELDS 9
 #define G2B_KERNEL_LAYER 1
 #define G2B_KERNEL_TILES 2

@@ -1,7 +1,7 @@
 """k_short over several spans of 128 positions, which calls take only under
-g2b_ctx_tune_kernel(3) (the automatic choice runs k_layer's splits past 128
-positions; below 128 positions k_short is a single span): each span of a (sequence, layer, KV head) writes its partials, the last to
-take a ticket merges them and writes the output; no combine launch.
+g2b_ctx_tune_kernel(3): each span of a (sequence, layer, KV head) writes its
+partials, the last to take a ticket merges them and writes the output; no
+combine launch.
 Against the oracle on the same seeded inputs: K and V bytes bit-exact,
 outputs within max-abs 1e-4 of float64 and of the oracle up to its own
 float32 error (helpers.check_out).  Every specialised shape, ragged
@@ -57,8 +57,7 @@ def test_qk_norm_vs_oracle(gpu_device, name):
 @pytest.mark.parametrize("q8", [True, False])
 def test_long_single_sequence(gpu_device, q8):
     """One sequence, layer by layer, at 20000 positions (157 spans, 1256
-    workgroups: more than one round, so the automatic choice would take
-    k_layer; asked for explicitly)."""
+    workgroups: more than one round)."""
     o = orc.Shape(2, 16, 8, 128, 1e6, orc.ARCH_QWEN3, q8)
     print(f"[spans] single sequence q8={q8}", flush=True)
     run_batch_case(o, [20001], [20000], seed=91, fused=False, want_att=False, kernel=3)
@@ -67,18 +66,17 @@ def test_long_single_sequence(gpu_device, q8):
 @pytest.mark.parametrize("q8", [True, False])
 def test_automatic_choice(gpu_device, q8):
     """Spans are taken only when asked for: the automatic choice for one layer
-    of one sequence past 128 positions (2049: 17 spans) is k_layer's static
-    splits, at least four per-lane wave-steps per wave, and the combine; below
-    128 positions it is a single span writing the output itself.  Outputs
-    against the oracle."""
+    of one sequence past 128 positions (2049: 17 spans) is k_wide's splits and
+    the combine, and up to 128 positions k_wide in one split that writes the
+    output itself.  Outputs against the oracle."""
     o = orc.Shape(1, 16, 8, 128, 1e6, orc.ARCH_QWEN3, q8)
     print(f"[spans] automatic q8={q8}", flush=True)
     sched = {}
     run_batch_case(o, [2049], [2048], seed=17, fused=False, want_att=False, sched=sched)
-    assert sched["kernel"] == "k_layer" and sched["max_splits"] > 1, sched
+    assert sched["kernel"] == "k_wide" and sched["max_splits"] > 1, sched
     assert not sched["output_in_kernel"], sched
     run_batch_case(o, [128], [127], seed=18, fused=False, want_att=False, sched=sched)
-    assert sched["kernel"] == "k_short" and sched["max_splits"] == 1, sched
+    assert sched["kernel"] == "k_wide" and sched["max_splits"] == 1, sched
     assert sched["output_in_kernel"], sched
 
 

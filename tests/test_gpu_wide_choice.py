@@ -40,4 +40,4 @@ def test_choice(gpu_device, name, poss, att, kernel):
     print(f"[choice] {name} {poss} att={att}", flush=True)
     sched = {}
     run_batch_case(o, caps, poss, seed=71, fused=False, want_att=att, sched=sched)
-    assert sched["variant"].startswith(kernel + "<"), sched
+    assert sched["kernel"] == kernel and sched["variant"].startswith(kernel + "<"), sched

@@ -37,7 +37,7 @@ def test_vs_oracle(gpu_device, name, poss, att, norm):
     sched = {}
     run_batch_case(o, caps, poss, seed=61, fused=len(poss) > 1, want_att=att, norms=norms, kernel=4,
                    sched=sched)
-    assert sched["variant"].startswith("k_wide<"), sched
+    assert sched["kernel"] == "k_wide" and sched["variant"].startswith("k_wide<"), sched
     whole = max(poss) < 128
     assert (sched["max_splits"] == 1) == whole, sched
     # (the weights are normalised by the combine)
