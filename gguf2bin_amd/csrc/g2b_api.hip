@@ -315,11 +315,15 @@ int32_t wide_split(const g2b_ctx *c, int64_t slots, int32_t n_seq, int64_t total
 //    -> 5.9, 126 positions 11.4 -> 8.7; 64 sequences of 50-103 14.7 -> 12.3, 256
 //    of them 35.8 -> 29.6 (9 / 3 of 64 14.6 -> 11.9); F32 rows of 4 KB 256 of
 //    50-103 (163 MB) 48.1 -> 47.3, but 256 of 64-127 (200 MB) 51.4 -> 52.3;
-//  - one layer of one sequence (k_layer; 32 / 8 of 128, Q8_0: k_tiles): Q8_0 at
-//    1000 13.9 -> 9.0, 8192 16.9 -> 15.5, 32767 33.3 -> 30.8; F32 at 2048 13.2 ->
-//    12.1, 32767 73 -> 54, but 8192 24.4 -> 26.4, 9000 24.7 -> 27.0 (splits cut
-//    for 16384 positions leave CUs idle; 11000 29.6 -> 28.1); 32 / 8, Q8_0 at
-//    1000 25.5 -> 9.1, 16383 28.6 -> 20.8, but 32767 30.2 -> 31.0;
+//  - one layer of one sequence (k_layer; 32 / 8 of 128, Q8_0: k_tiles), by its
+//    bucket alone (unit_positions), so that an eager step and a captured one of
+//    the bucket run the same kernel on the same splits: Q8_0 at 1000 13.9 ->
+//    9.0, 8192 16.9 -> 15.5, 32767 33.3 -> 30.8; F32 at 2048 13.2 -> 12.1, 16383
+//    37.5 -> 33.2, 32767 73 -> 54, but 8192 24.7 -> 27.5, 9000 25.1 -> 27.3, 10000
+//    26.1 -> 28.0 (splits cut for 16384 positions leave CUs idle; k_layer cut for
+//    them, as a captured step would be, 35.1, 35.2 and 35.0; 32 / 8 29.2 -> 28.0,
+//    27.4 -> 27.4, 28.6 -> 27.9); 32 / 8, Q8_0 at 1000 25.5 -> 9.1, 16383 28.6 ->
+//    20.8, but 32767 30.2 -> 31.0;
 //  - up to 64 units of at most 512 positions: 8 sequences of 150-303, Q8_0 20.2
 //    -> 11.4, 32 of 255-511 51.6 -> 20.6, 64 56.7 -> 43.8; F32 16 of 150-303 (30
 //    MB) 20.1 -> 16.3, but 32 of 255-511 29.4 -> 30.7;
@@ -337,8 +341,7 @@ bool wide_latency(const ShapeDev &sh, int32_t n_seq, int32_t n_layers, int32_t m
   const int64_t bytes = total_pos * n_layers * 2 * (int64_t)sh.row_bytes;
   const bool t = tiles_available(sh), f32_4k = !sh.kv_q8 && sh.row_bytes >= 4096;
   if (max_pos < kWideWhole) return !f32_4k || bytes <= 160 * kMB;
-  if (units == 1)
-    return t ? unit_positions(max_pos) <= 16384 : !(f32_4k && max_pos >= 8192 && max_pos < 10240);
+  if (units == 1) return !t || unit_positions(max_pos) <= 16384;
   if (units <= 64 && max_pos < 512) return !f32_4k || bytes <= 32 * kMB;
   return bytes <= (t ? 52 : 16) * kMB;
 }

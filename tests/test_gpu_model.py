@@ -148,6 +148,38 @@ def test_graph_replays_match_eager(gpu_device, tmp_path, kv_q8):
             assert np.array_equal(a.view(np.uint32), b.view(np.uint32)), f"step {i}"
 
 
+@pytest.mark.parametrize("heads,kv_q8", [((8, 8), False), ((16, 8), True), ((32, 8), True)])
+def test_graph_replays_match_eager_at_long_positions(gpu_device, tmp_path, heads, kv_q8):
+    """A replayed step of the bucket of 16384 positions gives the eager step's
+    logits bit for bit wherever in the bucket it lies (its first and last
+    positions, and those between): both run the same attention kernel on the
+    same splits.  The KV of the positions before is the device's seeded
+    fill, the same in both models."""
+    nh, nkv = heads
+    cfg = dict(dim=256, hidden_dim=256, n_layers=2, n_heads=nh, n_kv_heads=nkv, vocab=200,
+               seq_len=16384, head_dim=128, eps=1e-6, rope_theta=1e6)
+    rng = np.random.default_rng(nh + int(kv_q8))
+    p = str(tmp_path / "long.g2bx")
+    write_g2bx(p, cfg, attn.ARCH_QWEN3, F_QK_NORM,
+               random_model_slots(rng, cfg, F_QK_NORM, 8, 8, 8))
+    steps = [8192, 8193, 9000, 10239, 10240, 12345, 16383]
+    print(f"[model] long graph {heads} kv_q8={kv_q8}", flush=True)
+    with attn.Model(p, kv_q8=kv_q8) as g, attn.Model(p, kv_q8=kv_q8) as e:
+        g.use_graph(True)
+        e.use_graph(False)
+        for m in (g, e):
+            kc, vc, cap = m.kv()
+            ctx = attn.lib().g2b_model_ctx(m.h)
+            assert attn.lib().g2b_synth_fill_kv(ctx, kc, vc, cap, 0, 2, 0, cap, 77, 0,
+                                                float("inf")) == 0
+            assert attn.lib().g2b_sync(ctx) == 0
+        for pos in steps:
+            t = int(rng.integers(0, cfg["vocab"]))
+            a, b = g.forward(t, pos), e.forward(t, pos)
+            assert np.isfinite(a).all()
+            assert np.array_equal(a.view(np.uint32), b.view(np.uint32)), f"position {pos}"
+
+
 @pytest.mark.parametrize("name", ["qwen3_q8_tied", "llama_q4_f16emb", "mixed_types",
                                   "wide_dim_q4", "qwen3_q8_big_vocab", "qwen3_q8_mma_lm_head",
                                   "llama_q4_mma_lm_head"])

@@ -25,7 +25,7 @@ CASES = [
     ("qwen3_f32", [1023, 1023], False, "k_wide"),
     ("qwen3_f32", [1024, 1023], False, "k_layer"),
     ("qwen3_f32", [8191], False, "k_wide"),
-    ("qwen3_f32", [8192], False, "k_layer"),
+    ("qwen3_f32", [8192], False, "k_wide"),
     ("llama3_q8", [16383], False, "k_wide"),
     ("llama3_q8", [16384], False, "k_tiles"),
 ]
