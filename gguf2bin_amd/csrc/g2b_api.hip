@@ -309,8 +309,9 @@ int32_t wide_split(const g2b_ctx *c, int64_t slots, int32_t n_seq, int64_t total
 
 // Calls on k_layer's shapes that k_wide serves: those bound by latency, where
 // one KV head per workgroup and a setup that runs while the first tiles come
-// are shorter than k_short's and k_layer's chains, which cover all heads.  us
-// per layer, layer-serial, before -> k_wide (16 / 8 heads of 128 unless said):
+// are shorter than k_short's and k_layer's chains, which cover all heads.  A
+// unit is a layer of a sequence.  us per layer, layer-serial, before -> k_wide
+// (16 / 8 heads of 128 unless said; MB are 10^6 bytes, the lines MiB):
 //  - below kWideWhole positions, any batch (k_short): Q8_0 at 47 positions 8.6
 //    -> 5.9, 126 positions 11.4 -> 8.7; 64 sequences of 50-103 14.7 -> 12.3, 256
 //    of them 35.8 -> 29.6 (9 / 3 of 64 14.6 -> 11.9); F32 rows of 4 KB 256 of
@@ -333,17 +334,31 @@ int32_t wide_split(const g2b_ctx *c, int64_t slots, int32_t n_seq, int64_t total
 //    longer streams win (4 of 1500-3003, F32, 74 MB 24.0 -> 25.5; 64 of 750-1503,
 //    9 / 3, Q8_0, 29 MB 23.4 -> 25.5).  k_tiles has the longest setup: 16 of
 //    1000-2003, 32 / 8, Q8_0 (52 MB) 34.5 -> 29.0, 32 of 500-999 (52 MB) 68.8 ->
-//    29.5, 64 of 750-1503 (157 MB) 70.5 -> 101.6.
+//    29.5, 64 of 750-1503 (157 MB) 70.5 -> 101.6.  Not 33 to 47 units (21 to
+//    47 in a call over several layers), which within 16 MiB have 512 positions
+//    only where rows are short (9 / 3 of 64, Q8_0): there k_layer's splits end
+//    evenly and k_wide's do not: 40 sequences of 350-703 15.2 -> 16.9, of
+//    600-1203 17.2 -> 19.1 (of 450-903 18.0 -> 14.0); 32 of 350-703 15.2 -> 14.6,
+//    of 600-1203 16.9 -> 16.6, 28 15.9 -> 16.1, 48 of 350-703 15.2 -> 14.4.
+// Calls over several layers turn at the same lines (us per call, before ->
+// k_wide): below kWideWhole, 1 sequence x 28 layers of 47 9.0 -> 6.7, 64 x 28 of
+// 50-103 186 -> 150, F32 8 x 28 of 50-103 (141 MB) 33.7 -> 34.5, 64 x 4 (172 MB)
+// 39.7 -> 37.9; 1 x 28 of 503 20.4 -> 18.8, 2 x 28 of 250-503 57.0 -> 33.6, 32 / 8
+// 2 x 32 57.8 -> 23.6; 1 x 8 of 903 18.5 -> 16.5, 32 / 8 8 x 4 of 500-1003 (52
+// MB) 67.6 -> 26.9; 9 / 3, Q8_0, 1 x 20 of 1203 14.6 -> 13.1, 2 x 30 of 350-703
+// 17.3 -> 15.6, but 1 x 24 of 1203 14.8 -> 15.7, 1 x 30 of 1003 13.9 -> 16.0, 4 x 8
+// of 400-803 15.1 -> 16.1, 20 x 2 of 350-703 15.3 -> 17.1.
 bool wide_latency(const ShapeDev &sh, int32_t n_seq, int32_t n_layers, int32_t max_pos,
                   int64_t total_pos) {
-  constexpr int64_t kMB = 1 << 20;
+  constexpr int64_t kMiB = 1 << 20;
   const int64_t units = (int64_t)n_seq * n_layers;
   const int64_t bytes = total_pos * n_layers * 2 * (int64_t)sh.row_bytes;
   const bool t = tiles_available(sh), f32_4k = !sh.kv_q8 && sh.row_bytes >= 4096;
-  if (max_pos < kWideWhole) return !f32_4k || bytes <= 160 * kMB;
+  if (max_pos < kWideWhole) return !f32_4k || bytes <= 160 * kMiB;
   if (units == 1) return !t || unit_positions(max_pos) <= 16384;
-  if (units <= 64 && max_pos < 512) return !f32_4k || bytes <= 32 * kMB;
-  return bytes <= (t ? 52 : 16) * kMB;
+  if (units <= 64 && max_pos < 512) return !f32_4k || bytes <= 32 * kMiB;
+  if (t) return bytes <= 52 * kMiB;
+  return bytes <= 16 * kMiB && (units <= (n_layers == 1 ? 32 : 20) || units >= 48);
 }
 
 // Positions per split of a static schedule.  min_len is the shortest split

@@ -15,6 +15,7 @@ SHAPES = {
     "smollm2_q8": (9, 3, 64, orc.ARCH_LLAMA, True),
     "llama3_q8": (32, 8, 128, orc.ARCH_LLAMA, True),
 }
+# shape, positions, weights output, kernel[, layers in the one call]
 CASES = [
     ("qwen3_q8", [127], False, "k_wide"),
     ("qwen3_q8", [700], False, "k_wide"),
@@ -28,16 +29,29 @@ CASES = [
     ("qwen3_f32", [8192], False, "k_wide"),
     ("llama3_q8", [16383], False, "k_wide"),
     ("llama3_q8", [16384], False, "k_tiles"),
+    # units of up to 513 positions of 408 bytes: 20 and 21 in a call over several
+    # layers, 32, 33, 47 and 48 in one layer
+    ("smollm2_q8", [512, 64], False, "k_wide", 10),
+    ("smollm2_q8", [512, 64, 31], False, "k_layer", 7),
+    ("smollm2_q8", [512] + [40] * 31, False, "k_wide"),
+    ("smollm2_q8", [512] + [40] * 32, False, "k_layer"),
+    ("smollm2_q8", [512] + [40] * 46, False, "k_layer"),
+    ("smollm2_q8", [512] + [40] * 47, False, "k_wide"),
+    # rows of 4 KB, F32: 163840 KB of positions below 128 in one call are the line
+    ("qwen3_f32", [127] * 5, False, "k_wide", 32),
+    ("qwen3_f32", [127] * 5 + [0], False, "k_short", 32),
 ]
 
 
-@pytest.mark.parametrize("name,poss,att,kernel", CASES, ids=str)
-def test_choice(gpu_device, name, poss, att, kernel):
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "-".join(
+    [c[0], f"{len(c[1])}x{max(c[1])}", *map(str, c[2:])]))
+def test_choice(gpu_device, case):
+    (name, poss, att, kernel), layers = case[:4], case[4] if len(case) > 4 else 1
     nh, nkv, hd, arch, q8 = SHAPES[name]
-    o = orc.Shape(1, nh, nkv, hd, 1e5, arch, q8)
+    o = orc.Shape(layers, nh, nkv, hd, 1e5, arch, q8)
     # (rows of 204 bytes: whole capacities of eight rows keep caches aligned)
     caps = [(p // 8 + 1) * 8 for p in poss]
-    print(f"[choice] {name} {poss} att={att}", flush=True)
+    print(f"[choice] {name} {poss} att={att} layers={layers}", flush=True)
     sched = {}
-    run_batch_case(o, caps, poss, seed=71, fused=False, want_att=att, sched=sched)
+    run_batch_case(o, caps, poss, seed=71, fused=layers > 1, want_att=att, sched=sched)
     assert sched["kernel"] == kernel and sched["variant"].startswith(kernel + "<"), sched
