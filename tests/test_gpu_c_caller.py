@@ -22,8 +22,8 @@ EXE = os.path.join(HERE, "c_caller", "g2b_c_caller")
 
 CASES = {
     # name: (oracle shape, ctx_cap, tokens, with QK-RMSNorm)
-    # Qwen3 head shape, Q8_0 KV, QK-RMSNorm: k_short below 128 positions,
-    # the split kernel from 128 on
+    # Qwen3 head shape, Q8_0 KV, QK-RMSNorm: k_wide, the whole context in one
+    # split up to 128 positions, splits and a combine from there
     "qwen3_q8_qkn": (orc.Shape(2, 16, 8, 128, 1e6, orc.ARCH_QWEN3, True), 320, 300, True),
     # SmolLM2 head shape, F32 KV, LLaMA rotation
     "smollm2_f32": (orc.Shape(2, 9, 3, 64, 1e5, orc.ARCH_LLAMA, False), 200, 180, False),

@@ -134,10 +134,11 @@ def test_graph_replays_match_eager(gpu_device, tmp_path, kv_q8):
     scheduled for the step's own position; the synchronisation that ends
     every forward between the replays), each replay must give the eager
     step's logits bit for bit.  200 positions cover three buckets: 63 and
-    127, whose captured attention is k_short (as every eager step below 128
-    positions), and 255, whose captured attention is k_layer over two splits
-    and k_combine, replayed against eager steps at positions 128-199 (k_layer
-    with one or two splits: its own output, or k_combine)."""
+    127, whose captured attention is k_wide in one split that writes the
+    output (as every eager step below 128 positions), and 255, whose captured
+    attention is k_wide over splits of 64 positions and the combine, replayed
+    against eager steps at positions 128-199 (the same splits, fewer of
+    them)."""
     p, cfg, rng = make(tmp_path, "qwen3_hd128_q8", seed=5)
     toks = [int(t) for t in rng.integers(0, cfg["vocab"], 200)]
     with attn.Model(p, kv_q8=kv_q8) as g, attn.Model(p, kv_q8=kv_q8) as e:

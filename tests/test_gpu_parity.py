@@ -127,12 +127,16 @@ def test_codec_special_rows_on_device(gpu_device):
 
 
 @pytest.mark.parametrize("heads", [(2, 1, 64), (16, 8, 128)])
-def test_codec_special_rows_through_decode(gpu_device, heads):
+@pytest.mark.parametrize("kernel,tune,ran", [(0, None, "k_wide"), (1, None, "k_short"),
+                                             (1, (4, 0, -1, -1), "k_layer"),
+                                             (1, (4, 0, 2, -1), "k_layer")])
+def test_codec_special_rows_through_decode(gpu_device, heads, kernel, tune, ran):
     """The same quantiser branches through the append of a decode step (the
-    new row that the attention kernel itself quantises, four lanes per
-    block): row t of the special rows, tiled (and rolled) across nkv, is the
-    new k and v at pos t.  K and V bytes must equal the oracle's (reference
-    quantiser; K after RoPE at t)."""
+    new row that the attention kernel itself quantises: k_wide with four
+    elements per lane, k_short and k_layer four lanes per block): row t of
+    the special rows, tiled (and rolled) across nkv, is the new k and v at
+    pos t.  K and V bytes must equal the oracle's (reference quantiser; K
+    after RoPE at t)."""
     rows = q8_special_rows()
     nh, nkvh, hd = heads
     o = orc.Shape(1, nh, nkvh, hd, 1e4, orc.ARCH_QWEN3, True)
@@ -140,13 +144,17 @@ def test_codec_special_rows_through_decode(gpu_device, heads):
     tiled = np.stack([np.roll(np.tile(rows[t], nkv // 64), 7 * t) for t in range(n)])
     tiled = tiled.astype(np.float32)
     rng = np.random.default_rng(11)
-    print(f"[codec-decode] shape={o} rows={n}", flush=True)
+    print(f"[codec-decode] shape={o} rows={n} {ran}", flush=True)
     with attn.Context(ashape(o)) as ctx:
+        ctx.tune_kernel(kernel)
+        if tune:
+            ctx.tune(*tune)
         seq = DevSeq(ctx, o, n)
         try:
             for t in range(n):
                 q = rng.standard_normal(o.nq).astype(np.float32)
                 ctx.attn_forward_host(0, t, n, seq.k, seq.v, q, tiled[t], tiled[t])
+                assert ctx.last_schedule()["kernel"] == ran, ctx.last_schedule()
             kc, vc = seq.download()
         finally:
             seq.free()
@@ -172,8 +180,9 @@ SHAPES = {
     "f32_g1_hd128": (4, 4, 128, orc.ARCH_LLAMA, False),    # F32, G=1
     "tiny_q8_generic": (4, 2, 16, orc.ARCH_QWEN3, True),   # generic: blocks span heads
     "hd24_q8_generic": (4, 2, 24, orc.ARCH_QWEN3, True),   # generic: partial block
+    # (no k_layer: k_wide, or the generic kernels where q, k or v is unaligned)
     "hd256_f32_generic": (4, 2, 256, orc.ARCH_LLAMA, False),
-    "g8_q8_generic": (16, 2, 128, orc.ARCH_QWEN3, True),   # generic: group 8
+    "g8_q8_generic": (16, 2, 128, orc.ARCH_QWEN3, True),   # group 8
 }
 
 
@@ -204,7 +213,8 @@ def run_batch_case(o: orc.Shape, caps, poss, seed, fused: bool, want_att=True, n
     its inputs with them, and they are set on the context unless setup(ctx)
     is given to do that itself.  misalign: byte offset of q, k and v in their
     device buffers (not a multiple of 16: the generic kernels run).  kernel:
-    g2b_ctx_tune_kernel (0 automatic, 1 k_layer only).  sched: None or a
+    g2b_ctx_tune_kernel (0 automatic, 1 k_layer, or k_short below 128
+    positions, 2 k_tiles where it applies, 4 k_wide).  sched: None or a
     dict that receives the last call's schedule (g2b_ctx_last_schedule).
     q_gain: None or nq floats that multiply every q (outlier channels).
     w_as_accurate_as_ref: the weights' float64 bar (helpers.check_weights).
@@ -395,20 +405,23 @@ def test_static_grid_odd_splits_and_layer_rotation(gpu_device, name, split, stag
 
 @pytest.mark.parametrize("q8", [False, True])
 @pytest.mark.parametrize("norm", [False, True])
-def test_stepping_across_splits(gpu_device, q8, norm):
+@pytest.mark.parametrize("kernel", [0, 1])
+def test_stepping_across_splits(gpu_device, q8, norm, kernel):
     """A decode loop: one layer stepped one position per call from 120 to 200
-    on one context, each call appending its row (k_short below 128, then
-    k_layer's splits and the combine as their count grows; the first of
-    those calls allocates the context's buffers), every step against the
-    oracle; 8 query heads, 4 KV heads, head_dim 128, with and without
+    on one context, each call appending its row (automatic: k_wide in one
+    split up to 128 positions, then its splits and the combine; kernel 1:
+    k_short below 128, then k_layer's splits and the combine; the first of
+    the calls with a combine allocates the context's buffers), every step
+    against the oracle; 8 query heads, 4 KV heads, head_dim 128, with and without
     QK-RMSNorm."""
     o = orc.Shape(1, 8, 4, 128, 1e6, orc.ARCH_QWEN3, q8)
     cap, eps = 256, 1e-6
     rng = np.random.default_rng(7 + 2 * int(q8) + int(norm))
     qn = (1 + 0.25 * rng.standard_normal(o.head_dim)).astype(np.float32) if norm else None
     kn = (1 + 0.25 * rng.standard_normal(o.head_dim)).astype(np.float32) if norm else None
-    print(f"[stepping] q8={q8} norm={norm}", flush=True)
+    print(f"[stepping] q8={q8} norm={norm} kernel={kernel}", flush=True)
     with attn.Context(ashape(o)) as ctx:
+        ctx.tune_kernel(kernel)
         if norm:
             ctx.set_qk_norm(0, qn, kn, eps)
         kc, vc = ctx.kv_alloc(cap)
@@ -428,6 +441,8 @@ def test_stepping_across_splits(gpu_device, q8, norm):
                 qd, kk, vv = hip.to_device(q), hip.to_device(k), hip.to_device(v)
                 ctx.attn_forward(0, pos, cap, kc, vc, qd.ptr, kk.ptr, vv.ptr)
                 ctx.sync()
+                ran = "k_wide" if kernel == 0 else "k_short" if pos < 128 else "k_layer"
+                assert ctx.last_schedule()["kernel"] == ran, ctx.last_schedule()
                 out = qd.download(np.float32, q.size)
                 ql = normed(q, qn, o.n_heads, o.head_dim, eps)
                 kl = normed(k, kn, o.n_kv_heads, o.head_dim, eps)
@@ -454,10 +469,12 @@ SHORT_SHAPES = sorted(n for n in SHAPES if "generic" not in n)
 
 @pytest.mark.parametrize("name", SHORT_SHAPES)
 @pytest.mark.parametrize("norm", ["none", "qk"])
-def test_short_contexts_vs_oracle(gpu_device, name, norm):
-    """Every pos below 128 and no weights output: the short-context kernel
-    (one workgroup per KV head, sequence and layer; output written over q,
-    no combine) - outputs within the bars and K/V bytes bit-exact against
+@pytest.mark.parametrize("kernel,ran", [(0, "k_wide"), (1, "k_short")])
+def test_short_contexts_vs_oracle(gpu_device, name, norm, kernel, ran):
+    """Every pos below 128 and no weights output: k_wide in one split (the
+    automatic choice) and the short-context kernel (both one workgroup per KV
+    head, sequence and layer; output written over q, no combine) - outputs
+    within the bars and K/V bytes bit-exact against
     the oracle, all layers in one call and layer by layer, pos 0 and 127
     (the last position it takes) included; then the same inputs through the
     split kernel (an explicit split length of 64 keeps it)."""
@@ -470,12 +487,17 @@ def test_short_contexts_vs_oracle(gpu_device, name, norm):
         kn = (1 + 0.25 * orc.normal(seed + 41, 2 * hd)).reshape(2, hd)
         norms = (qn, kn, 1e-6)
     caps, poss = [1, 2, 37, 128, 129], [0, 1, 36, 127, 64]
-    print(f"[short] {name} norm={norm}", flush=True)
-    a = run_batch_case(o, caps, poss, seed, fused=True, want_att=False, norms=norms)
-    b = run_batch_case(o, caps, poss, seed, fused=False, want_att=False, norms=norms)
+    print(f"[short] {name} norm={norm} {ran}", flush=True)
+    sa, sb, sc = {}, {}, {}
+    a = run_batch_case(o, caps, poss, seed, fused=True, want_att=False, norms=norms,
+                       kernel=kernel, sched=sa)
+    b = run_batch_case(o, caps, poss, seed, fused=False, want_att=False, norms=norms,
+                       kernel=kernel, sched=sb)
+    assert sa["kernel"] == sb["kernel"] == ran, (sa, sb)
     assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
     run_batch_case(o, caps, poss, seed, fused=True, want_att=False, norms=norms,
-                   tune=(64, 0, 0, 0))
+                   kernel=kernel, tune=(64, 0, 0, 0), sched=sc)
+    assert sc["kernel"] in ("k_layer", "k_tiles") and sc["max_splits"] == 2, sc
 
 
 QKN_SHAPES = {

@@ -6,8 +6,10 @@ oracle up to the oracle's own float32 error (helpers.check_out; the oracle is
 bit-exact with the compiled reference on the golden cases).  Every schedule
 (static splits, the work queue, one call over all layers, layer by layer),
 partial tiles and pieces, QK-RMSNorm, and the c5 shape at full context
-length through the work queue.  k_layer runs the same cases
-(g2b_ctx_tune_kernel(1)) so both kernels keep their coverage."""
+length through the work queue.  g2b_ctx_tune_kernel(2) asks for k_tiles (the
+automatic choice gives those of these calls that latency bounds to k_wide);
+k_layer runs the same cases (g2b_ctx_tune_kernel(1)) so both kernels keep
+their coverage."""
 import zlib
 
 import numpy as np
@@ -27,6 +29,8 @@ TILE_SHAPES = {
     "g3": (24, 8, orc.ARCH_QWEN3),
 }
 
+KERNEL = {1: "k_layer", 2: "k_tiles"}  # what g2b_ctx_tune_kernel asks for
+
 
 def oshape(name, layers=2):
     nh, nkv, arch = TILE_SHAPES[name]
@@ -35,21 +39,23 @@ def oshape(name, layers=2):
 
 @pytest.mark.parametrize("name", sorted(TILE_SHAPES))
 @pytest.mark.parametrize("mode", ["fused", "layers", "wq", "wq_fused", "static"])
-@pytest.mark.parametrize("kernel", [0, 1])
+@pytest.mark.parametrize("kernel", [2, 1])
 def test_ragged_batch_vs_oracle(gpu_device, name, mode, kernel):
     """Ragged sequences (pos 0, 1, mid-tile, a whole number of tiles, long):
-    no weights output, so k_tiles runs unless kernel 1 asks for k_layer."""
+    no weights output, so k_tiles runs under kernel 2, k_layer under 1."""
     o = oshape(name)
     fused, tune = MODES[mode]
     caps = [1, 2, 40, 129, 700, 2049]
     poss = [0, 1, 39, 128, 650, 2048]
     print(f"[tiles] {name} mode={mode} kernel={kernel}", flush=True)
+    sched = {}
     run_batch_case(o, caps, poss, seed=zlib.crc32(name.encode()) % 1000, fused=fused,
-                   want_att=False, tune=tune, kernel=kernel)
+                   want_att=False, tune=tune, kernel=kernel, sched=sched)
+    assert sched["kernel"] == KERNEL[kernel], sched
 
 
 @pytest.mark.parametrize("name", sorted(TILE_SHAPES))
-@pytest.mark.parametrize("kernel", [0, 1])
+@pytest.mark.parametrize("kernel", [2, 1])
 def test_qk_norm_vs_oracle(gpu_device, name, kernel):
     o = oshape(name)
     hd = o.head_dim
@@ -57,8 +63,10 @@ def test_qk_norm_vs_oracle(gpu_device, name, kernel):
     qn = (1 + 0.25 * orc.normal(seed + 40, 2 * hd)).reshape(2, hd)
     kn = (1 + 0.25 * orc.normal(seed + 41, 2 * hd)).reshape(2, hd)
     print(f"[tiles] qknorm {name} kernel={kernel}", flush=True)
+    sched = {}
     run_batch_case(o, [1, 37, 300, 129], [0, 36, 211, 64], seed=seed, fused=False,
-                   want_att=False, norms=(qn, kn, 1e-5), kernel=kernel)
+                   want_att=False, norms=(qn, kn, 1e-5), kernel=kernel, sched=sched)
+    assert sched["kernel"] == KERNEL[kernel], sched
 
 
 @pytest.mark.parametrize("mode", ["layers", "wq"])
@@ -68,8 +76,10 @@ def test_many_tiles_single_sequence(gpu_device, mode):
     partial."""
     o = oshape("llama3_g4", layers=1)
     print(f"[tiles] single sequence mode={mode}", flush=True)
+    sched = {}
     run_batch_case(o, [6000], [5999], seed=78, fused=False, want_att=False,
-                   tune=(0, 0, 2, 12) if mode == "wq" else None)
+                   tune=(0, 0, 2, 12) if mode == "wq" else None, kernel=2, sched=sched)
+    assert sched["kernel"] == "k_tiles", sched
 
 
 def test_weights_output_takes_layer_kernel(gpu_device):
@@ -77,7 +87,9 @@ def test_weights_output_takes_layer_kernel(gpu_device):
     writes no raw scores); outputs and weights within the bars."""
     o = oshape("llama3_g4")
     print("[tiles] weights output", flush=True)
-    run_batch_case(o, [1, 300, 129], [0, 211, 64], seed=9, fused=True, want_att=True)
+    sched = {}
+    run_batch_case(o, [1, 300, 129], [0, 211, 64], seed=9, fused=True, want_att=True, sched=sched)
+    assert sched["kernel"] == "k_layer", sched
 
 
 @pytest.mark.parametrize("fused", [False, True])

@@ -12,10 +12,10 @@ from test_gpu_parity import run_batch_case
 
 pytestmark = pytest.mark.gpu
 
-# n_heads, n_kv_heads, head_dim, arch, q8: groups of 1 to 16 (one, two and
-# four sets of four heads, full and ragged), one to four KV heads per
-# workgroup, one or several workgroups per split, rows that are not whole
-# 16-byte pieces (136 bytes)
+# n_heads, n_kv_heads, head_dim, arch, q8: every instance (both formats, head
+# sizes 64, 128 and 256, one, two and four sets of four heads, full and ragged
+# groups of 1 to 16), one to twenty KV heads (a workgroup each), rows that are
+# not whole 16-byte pieces (136 and 68 bytes)
 SHAPES = {
     "g5_hd64_q8": (10, 2, 64, orc.ARCH_LLAMA, True),
     "g7_hd64_f32": (14, 2, 64, orc.ARCH_QWEN3, False),
@@ -26,9 +26,15 @@ SHAPES = {
     "mha20_hd128_q8": (20, 20, 128, orc.ARCH_LLAMA, True),
     "g6_hd256_q8": (12, 2, 256, orc.ARCH_QWEN3, True),
     "g2_hd256_f32": (8, 4, 256, orc.ARCH_LLAMA, False),
+    "mqa16_hd64_q8": (16, 1, 64, orc.ARCH_LLAMA, True),
+    "g12_hd64_f32": (24, 2, 64, orc.ARCH_QWEN3, False),
+    "g4_hd256_q8": (8, 2, 256, orc.ARCH_LLAMA, True),
+    "g16_hd256_q8": (32, 2, 256, orc.ARCH_QWEN3, True),
+    "g8_hd256_f32": (16, 2, 256, orc.ARCH_QWEN3, False),
+    "g9_hd256_f32": (9, 1, 256, orc.ARCH_LLAMA, False),
 }
-# positions at the edges of a tile (16), of the tiles of 1, 2 and 4 waves and
-# of splits, from the first position on
+# positions at the edges of a tile (16), of a round of four waves' tiles (64)
+# and of splits, from the first position on
 POS = [0, 1, 15, 16, 17, 63, 64, 150]
 
 
@@ -50,6 +56,21 @@ def test_wide_vs_oracle(gpu_device, name, split, att, norm):
                        sched=sched)
         assert sched["kernel"] == "k_wide", sched
         assert not split or sched["split_len"] == min(split, max(poss) + 1), sched
+
+
+@pytest.mark.parametrize("name", ["g8_hd128_q8", "mha20_hd128_q8", "g9_3kv_hd128_f32",
+                                  "g16_hd256_q8", "g9_hd256_f32", "mqa16_hd64_q8"])
+def test_wide_ragged_batch(gpu_device, name):
+    """20 sequences of 1 to 2500 positions: the splits of a batch, of every
+    length down to none, and partials of several rounds in the combine."""
+    nh, nkv, hd, arch, q8 = SHAPES[name]
+    o = orc.Shape(1, nh, nkv, hd, 1e5, arch, q8)
+    poss = [(2499 * i * i) // 361 for i in range(20)]
+    print(f"[wide] ragged batch {name}", flush=True)
+    sched = {}
+    run_batch_case(o, [p + 1 for p in poss], poss, seed=23, fused=False, want_att=False,
+                   sched=sched)
+    assert sched["kernel"] == "k_wide", sched
 
 
 def test_wide_outlier_q(gpu_device):

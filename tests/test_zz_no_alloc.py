@@ -21,18 +21,32 @@ from gguf2bin_amd import attn, hip
 pytestmark = pytest.mark.gpu
 
 CASES = {
-    # name: (oracle shape, ctx_cap, positions of the two calls, same splits as forward?)
-    # k_layer, static splits
-    "qwen3_q8": (orc.Shape(1, 16, 8, 128, 1e6, orc.ARCH_QWEN3, True), 6000, (5999, 700), True),
+    # name: (oracle shape, ctx_cap, positions of the two calls, same splits as forward?,
+    #        g2b_ctx_tune_kernel, the kernel that runs)
+    # k_wide and k_layer, static splits
+    "qwen3_q8": (orc.Shape(1, 16, 8, 128, 1e6, orc.ARCH_QWEN3, True), 6000, (5999, 700), True,
+                 0, "k_wide"),
+    "qwen3_q8_layer": (orc.Shape(1, 16, 8, 128, 1e6, orc.ARCH_QWEN3, True), 6000, (5999, 700),
+                       True, 1, "k_layer"),
     # k_tiles, static splits; the first call's splits are lengthened to fit
     "llama3_q8_long": (orc.Shape(1, 32, 8, 128, 5e5, orc.ARCH_LLAMA, True), 32768,
-                       (32767, 4000), False),
+                       (32767, 4000), False, 2, "k_tiles"),
     # F32 rows
-    "smollm2_f32": (orc.Shape(1, 9, 3, 64, 1e5, orc.ARCH_LLAMA, False), 3000, (2999, 500), True),
+    "smollm2_f32": (orc.Shape(1, 9, 3, 64, 1e5, orc.ARCH_LLAMA, False), 3000, (2999, 500), True,
+                    0, "k_wide"),
+    "smollm2_f32_layer": (orc.Shape(1, 9, 3, 64, 1e5, orc.ARCH_LLAMA, False), 3000, (2999, 500),
+                          True, 1, "k_layer"),
+    # a shape that only k_wide and the generic kernels take
+    "group8_q8": (orc.Shape(1, 16, 2, 128, 1e6, orc.ARCH_QWEN3, True), 3000, (2999, 40), True,
+                  0, "k_wide"),
     # the generic kernels (rotated q in the scratch too)
-    "generic_hd24": (orc.Shape(1, 4, 2, 24, 1e4, orc.ARCH_QWEN3, True), 3000, (2999, 40), True),
-    # the short-context kernel: no scratch at all
-    "short": (orc.Shape(1, 16, 8, 128, 1e6, orc.ARCH_QWEN3, True), 200, (120, 10), True),
+    "generic_hd24": (orc.Shape(1, 4, 2, 24, 1e4, orc.ARCH_QWEN3, True), 3000, (2999, 40), True,
+                     0, "k_decode_generic"),
+    # short contexts: no scratch at all
+    "short": (orc.Shape(1, 16, 8, 128, 1e6, orc.ARCH_QWEN3, True), 200, (120, 10), True,
+              0, "k_wide"),
+    "short_kernel": (orc.Shape(1, 16, 8, 128, 1e6, orc.ARCH_QWEN3, True), 200, (120, 10), True,
+                     1, "k_short"),
 }
 
 
@@ -43,13 +57,14 @@ def ashape(o):
 
 @pytest.mark.parametrize("name", sorted(CASES))
 def test_noalloc_matches_allocating_entry_point(gpu_device, name):
-    o, cap, calls, same = CASES[name]
+    o, cap, calls, same, tune_kernel, kernel = CASES[name]
     rng = np.random.default_rng(sum(map(ord, name)))
     n_pre = calls[0]
     kp = rng.standard_normal((n_pre, o.nkv)).astype(np.float32)
     vp = rng.standard_normal((n_pre, o.nkv)).astype(np.float32)
     nbytes = attn.kv_bytes(ashape(o), cap)
     with attn.Context(ashape(o)) as ctx:
+        ctx.tune_kernel(tune_kernel)
         a, b = ctx.kv_alloc(cap), ctx.kv_alloc(cap)  # forward's caches, noalloc's caches
         host = orc.alloc_kv(o, cap)
         try:
@@ -68,6 +83,7 @@ def test_noalloc_matches_allocating_entry_point(gpu_device, name):
                 ctx.attn_forward(0, pos, cap, a[0], a[1], qa.ptr, kk.ptr, vv.ptr)
                 ctx.attn_forward_noalloc(0, pos, cap, b[0], b[1], qb.ptr, kk.ptr, vv.ptr)
                 ctx.sync()
+                assert ctx.last_schedule()["kernel"] == kernel, ctx.last_schedule()
                 out_a = qa.download(np.float32, o.nq)
                 out_b = qb.download(np.float32, o.nq)
                 ref, _ = orc.attn_layer(o, cap, 0, pos, host[0], host[1], q, k, v)
@@ -103,11 +119,11 @@ def test_noalloc_refusals(gpu_device):
             assert e.value.code == attn.G2B_EPOS
         finally:
             owner.kv_free(kc, vc)
-    # a shape without a specialised kernel (group 8: the generic kernels, at
-    # most 1024 positions per split): one split is 16 x 132 floats of
-    # partials, so the 2 MiB scratch (524,288 floats, after the 1024 counter
-    # words and the 2048 floats of rotated q) holds 246 splits, 251,904
-    # positions; 259,999 need longer splits than the kernel takes
+    # a shape of k_wide and the generic kernels (group 8), whose bounds are the
+    # generic ones' for both (at most 1024 positions per split): one split is
+    # 16 x 132 floats of partials, so the 2 MiB scratch (524,288 floats, after
+    # the 1024 counter words and the 2048 floats of rotated q) holds 246
+    # splits, 251,904 positions; 259,999 need longer splits
     big = attn.Shape(1, 16, 2, 128, 1e6, attn.ARCH_QWEN3, True)
     with attn.Context(big) as ctx:
         kc, vc = ctx.kv_alloc(260000)
@@ -125,8 +141,8 @@ def test_noalloc_refusals(gpu_device):
 
 def test_noalloc_allocates_nothing_and_replays_from_a_graph(gpu_device):
     """hipMemGetInfo around the first g2b_attn_forward_noalloc of a context
-    that has only allocated its KV (k_layer's static splits: 50 splits of
-    partials in the fixed scratch), then the same call captured on the
+    that has only allocated its KV (k_wide's splits, their partials in the
+    fixed scratch), then the same call captured on the
     context's stream and replayed three times, with eager calls and
     synchronisations between the replays, each replay bit for bit equal to
     the direct call (the append at pos rewrites the same bytes)."""
