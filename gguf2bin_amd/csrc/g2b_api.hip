@@ -235,13 +235,6 @@ int ensure_rope(g2b_ctx *c, int32_t len) {
   return G2B_OK;
 }
 
-// Positions per split.  The decode workgroups of one call should form whole
-// rounds of the device's resident slots (CUs x workgroups per CU): with equal
-// work per workgroup they start and finish together, and the launch has no
-// partly idle tail.  One round when the work allows it; otherwise as many
-// rounds as the minimum split length forces.  At most 512 splits per
-// sequence (each is one partial per head for the combine, which stages a
-// weight per partial in LDS) and the generic kernel's LDS limit apply.
 // Resident k_layer workgroups on the device for the variant of dp (cached).
 int32_t slots_for(g2b_ctx *c, const DecodeParams &dp, bool wq) {
   int32_t &occ = c->occ_cache[dp.tune_chunk == 16 ? 1 : 0][dp.stage_mode][wq ? 1 : 0];
@@ -361,7 +354,14 @@ bool wide_latency(const ShapeDev &sh, int32_t n_seq, int32_t n_layers, int32_t m
   return bytes <= 16 * kMiB && (units <= (n_layers == 1 ? 32 : 20) || units >= 48);
 }
 
-// Positions per split of a static schedule.  min_len is the shortest split
+// Positions per split of a static schedule of k_layer, k_tiles or the generic
+// kernel.  The decode workgroups of one call should form whole rounds of the
+// device's resident slots (CUs x workgroups per CU): with equal work per
+// workgroup they start and finish together, and the launch has no partly idle
+// tail.  One round when the work allows it; otherwise as many rounds as the
+// minimum split length forces.  At most 512 splits per sequence (each is one
+// partial per head for the combine, which stages a weight per partial in LDS)
+// and the generic kernel's LDS limit apply.  min_len is the shortest split
 // worth a workgroup (its waves get a few wave-steps or chunks each; shorter
 // splits cost more in setup and partials than they gain).
 //
@@ -595,6 +595,8 @@ int run_layers(g2b_ctx *c, const SeqDev *d_seqs, const SeqDev &one, int32_t n_se
   // per-lane loads, whose first trip is in flight during the setup (c2, 8193
   // positions: 545 us per layer-serial step against 580 us for staged
   // chunks).
+  // (k_layer sees one unit with the weights output or a tuning only: without,
+  // k_wide runs it, or k_tiles past 16384 positions of its shapes)
   const bool one_unit = n_seq == 1 && n_layers == 1;
   dp.stage_mode = c->tune_stage < 0   ? 0
                   : c->tune_stage > 0 ? c->tune_stage
@@ -626,7 +628,8 @@ int run_layers(g2b_ctx *c, const SeqDev *d_seqs, const SeqDev &one, int32_t n_se
   }
 
   // k_short, no weights output, where k_wide is not taken (a tuning, or F32
-  // rows of 4 KB in large batches): one workgroup per (KV head, span of kShortMaxPos positions, sequence, layer).  Below kShortMaxPos positions
+  // rows of 4 KB in large batches): one workgroup per (KV head, span of
+  // kShortMaxPos positions, sequence, layer).  Below kShortMaxPos positions
   // it is a single span that writes the output over q itself.  Longer
   // contexts take it (spans that merge their partials in the kernel, no
   // combine launch) only when g2b_ctx_tune_kernel(3) asks for it: one layer

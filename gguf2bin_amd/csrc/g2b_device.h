@@ -175,6 +175,13 @@ __device__ __forceinline__ float half_bits_to_f32_hw(uint32_t h) {
   return (float)__builtin_bit_cast(_Float16, (uint16_t)h);
 }
 
+// Where piece p (elements 4p .. 4p + 3) of an x of nb 32-element blocks lies
+// in LDS, in float4s: piece j of every block together, block by block.  The
+// GEMVs' lanes read piece j of consecutive blocks in one instruction, which
+// this order serves from consecutive addresses; as x lies in memory they are
+// 128 bytes apart, on the same four banks.
+__device__ __forceinline__ int gemv_x_piece(int nb, int p) { return (p & 7) * nb + (p >> 3); }
+
 // sum(x[i]^2), i < n, over a workgroup of 256 threads (x 16-byte aligned;
 // red: 4 floats of LDS), returned to every thread: thread t accumulates the
 // float4 pieces t, t + 256, ... in element order (eight loads in flight),
@@ -183,12 +190,6 @@ __device__ __forceinline__ float half_bits_to_f32_hw(uint32_t h) {
 // order; one order for every kernel that normalises, so they agree bitwise.
 // STAGE: also x[i] * w[i] into xw (LDS; n a multiple of 32) in gemv_x_piece's
 // order.
-// Where piece p (elements 4p .. 4p + 3) of an x of nb 32-element blocks lies
-// in LDS, in float4s: piece j of every block together, block by block.  The
-// GEMVs' lanes read piece j of consecutive blocks in one instruction, which
-// this order serves from consecutive addresses; as x lies in memory they are
-// 128 bytes apart, on the same four banks.
-__device__ __forceinline__ int gemv_x_piece(int nb, int p) { return (p & 7) * nb + (p >> 3); }
 template <bool STAGE>
 __device__ inline float wg256_sumsq_t(const float *x, int n, float *red, const float *w,
                                       float *xw) {

@@ -248,10 +248,11 @@ constexpr int kTilesRows = 16;
 bool tiles_available(const ShapeDev &sh);
 hipError_t launch_tiles(const DecodeParams &p, int n_layers, hipStream_t s);
 int tiles_blocks_per_cu(const ShapeDev &sh, bool wq);
-// Shapes neither k_layer nor k_tiles takes, with head_dim 64, 128 or 256 and
-// up to 16 q heads per KV head: k_wide (g2b_wide.h) does RoPE, append and
-// attention with both products on the matrix cores; static splits, partials
-// as k_layer's.
+// head_dim 64, 128 or 256 and up to 16 q heads per KV head: k_wide
+// (g2b_wide.h) does RoPE, append and attention with both products on the
+// matrix cores; static splits, partials as k_layer's.  It runs the shapes
+// that neither k_layer nor k_tiles takes and, of theirs, the calls that
+// latency bounds (wide_latency in g2b_api.hip).
 bool wide_available(const ShapeDev &sh);
 hipError_t launch_wide(const DecodeParams &p, int n_layers, hipStream_t s);
 // Its resident workgroups per CU (a split is one per KV head), and the

@@ -711,8 +711,7 @@ __device__ inline void visit_setup(const ShapeDev &sh, const SeqDev &sd, int lay
   if (!DIG && !owns_new) return;  // qrot was published by the barrier above
   __syncthreads();
   if (!owns_new) return;
-  const size_t off =
-      ((size_t)layer * (size_t)sd.ctx_cap + (size_t)sd.pos) * sh.row_bytes;
+  const size_t off = ((size_t)layer * (size_t)sd.ctx_cap + (size_t)sd.pos) * sh.row_bytes;
   uint32_t *gk = reinterpret_cast<uint32_t *>(sd.k + off);
   uint32_t *gv = reinterpret_cast<uint32_t *>(sd.v + off);
   const uint32_t *lk = reinterpret_cast<const uint32_t *>(rowk);

@@ -1105,14 +1105,17 @@ hipError_t launch_rows_k(GemvParams p, int n_cu, hipStream_t s) {
   // 3072 rows of 1024 Q8_0 weights 3.1 us either way, 6144 rows 3.7 us in 768
   // workgroups of single steps, 3.9 us in 384 of pairs.
   const bool two = p.steps > 3 * wpw * n_cu;
+  // (resident workgroups with the longest x that the instance takes: one
+  // figure for every call, whatever x came first)
+  constexpr size_t most = (size_t)LPR * KB * 128u;
   int &o = occ[two ? 1 : 0];
   if (o == 0) {
     int n = 0;
     const hipError_t e =
         two ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_gemv_rows<FMT, LPR, KB, 2>,
-                                                           kGemvThreads, x_lds(p))
+                                                           kGemvThreads, most)
             : hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_gemv_rows<FMT, LPR, KB, 1>,
-                                                           kGemvThreads, x_lds(p));
+                                                           kGemvThreads, most);
     if (e != hipSuccess || n < 1) {
       (void)hipGetLastError();
       n = 1;

@@ -214,12 +214,6 @@ __device__ __forceinline__ float wave_max(float x) {
   return x;
 }
 
-__device__ __forceinline__ float wave_sum(float x) {
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) x += __shfl_xor(x, o);
-  return x;
-}
-
 #ifdef G2B_STAMPS
 // Phase stamps of a k_short workgroup (thread 0; one-span calls): 0 entry,
 // 1 inputs and the norm factors in, 2 RoPE done, 3 append done, 4 scores
