@@ -17,19 +17,12 @@ __device__ __forceinline__ float dpp_f(float x) {
   return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), CTRL, 0xF, 0xF, true));
 }
 
-template <int CTRL>
-__device__ __forceinline__ uint32_t dpp_u(uint32_t x) {
-  return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, CTRL, 0xF, 0xF, true);
+// The larger of m and |x|, NaN if either is (gfx950's v_maximum3_f32; fmaxf
+// loses a NaN), and whether the largest of several is finite.
+__device__ __forceinline__ float max_abs(float m, float x) {
+  return __builtin_elementwise_maximum(m, fabsf(x));
 }
-
-// |x| as bits, for the largest of several: as unsigned integers finite |x|
-// lie in their own order, Inf above them and NaN above Inf, so a maximum at
-// or above kInfBits says that a non-finite x was among them (fmaxf loses a
-// NaN).
-constexpr uint32_t kInfBits = 0x7f800000u;
-__device__ __forceinline__ uint32_t abs_bits(float x) {
-  return __float_as_uint(x) & 0x7fffffffu;
-}
+__device__ __forceinline__ bool finite_max(float m) { return m <= 3.402823466e38f; }
 
 // Sum over aligned groups of N consecutive lanes; every lane of a group ends
 // with the same value (each step adds two equal-order operands).

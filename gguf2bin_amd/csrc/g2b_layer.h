@@ -305,27 +305,27 @@ __device__ __forceinline__ void split_digits(int m, int (&d)[kQPlanes]) {
   d[kQPlanes - 1] = m;
 }
 
-// 2^(kQBits-e) and 2^(e-kQBits) of a chunk whose largest |q| has the bits mx
-// (abs_bits).  A chunk that holds an Inf or a NaN has no digits: they are 0
+// 2^(kQBits-e) and 2^(e-kQBits) of a chunk whose largest |q| (max_abs) is mx.
+// A chunk that holds an Inf or a NaN has no digits: they are 0
 // and the unit is NaN, so every score of its head, and with them the head's
 // output, is NaN, as in the fp32 dot (Inf in q meets both signs of k; the
 // softmax of infinite scores is NaN).
 struct DigitScale {
   float up, unit;
 };
-__device__ __forceinline__ DigitScale digit_scale(uint32_t mx) {
+__device__ __forceinline__ DigitScale digit_scale(float mx) {
   int e = 0;
-  (void)frexpf(__uint_as_float(mx), &e);
-  if (mx >= kInfBits) return {0.f, __int_as_float(0x7fc00000)};
+  (void)frexpf(mx, &e);
+  if (!finite_max(mx)) return {0.f, __int_as_float(0x7fc00000)};
   return {ldexpf(1.f, kQBits - e), ldexpf(1.f, e - kQBits)};
 }
 
 template <int CD>
 __device__ __forceinline__ QDigits<CD> make_digits(const float (&q)[CD]) {
   QDigits<CD> r;
-  uint32_t mx = 0u;
+  float mx = 0.f;
 #pragma unroll
-  for (int j = 0; j < CD; j++) mx = max(mx, abs_bits(q[j]));
+  for (int j = 0; j < CD; j++) mx = max_abs(mx, q[j]);
   const DigitScale ds = digit_scale(mx);
   r.unit = ds.unit;
 #pragma unroll
@@ -661,11 +661,11 @@ __device__ inline void visit_setup(const ShapeDev &sh, const SeqDev &sd, int lay
         q[j + 2] = v4.z * qscale;
         q[j + 3] = v4.w * qscale;
       }
-      uint32_t mx = 0u;
+      float mx = 0.f;
 #pragma unroll
-      for (int j = 0; j < QE; j++) mx = max(mx, abs_bits(q[j]));
-      mx = max(mx, (uint32_t)__shfl_xor((int)mx, 1));
-      mx = max(mx, (uint32_t)__shfl_xor((int)mx, 2));
+      for (int j = 0; j < QE; j++) mx = max_abs(mx, q[j]);
+      mx = max_abs(mx, __shfl_xor(mx, 1));
+      mx = max_abs(mx, __shfl_xor(mx, 2));
       const DigitScale ds = digit_scale(mx);
       uint32_t d[kQPlanes][QE / 4];
 #pragma unroll

@@ -272,12 +272,12 @@ __device__ __forceinline__ void lane_x(const GemvParams &P, const float *xs, int
   }
 }
 
-// The largest |x| of a block, as bits (abs_bits: Inf and NaN lie at and above
-// kInfBits), from the four elements that each of its eight lanes holds.
-__device__ __forceinline__ uint32_t block_abs_bits(const float4 &v) {
-  uint32_t mx = max(max(abs_bits(v.x), abs_bits(v.y)), max(abs_bits(v.z), abs_bits(v.w)));
+// The largest |x| of a block (NaN if one is), from the four elements that each
+// of its eight lanes holds.
+__device__ __forceinline__ float block_max_abs(const float4 &v) {
+  float mx = max_abs(max_abs(max_abs(fabsf(v.x), v.y), v.z), v.w);
 #pragma unroll
-  for (int o = 1; o < 8; o *= 2) mx = max(mx, (uint32_t)__shfl_xor((int)mx, o));
+  for (int o = 1; o < 8; o *= 2) mx = max_abs(mx, __shfl_xor(mx, o));
   return mx;
 }
 
@@ -301,9 +301,9 @@ __device__ __forceinline__ void wg_x_digits(const GemvParams &P, const float *xs
     const int b = it >> 3, j = it & 7;  // chunk j: elements 4j .. 4j+3 of block b
     const float4 v = P.pro == kProNone ? reinterpret_cast<const float4 *>(P.x)[it]
                                        : staged_x4(P, xs, b, j, inv);
-    const uint32_t mx = block_abs_bits(v);
+    const float mx = block_max_abs(v);
     int e = 0;
-    (void)frexpf(__uint_as_float(mx), &e);
+    (void)frexpf(mx, &e);
     const float xv[4] = {v.x, v.y, v.z, v.w};
     uint32_t pl[4] = {0u, 0u, 0u, 0u};
 #pragma unroll
@@ -323,7 +323,7 @@ __device__ __forceinline__ void wg_x_digits(const GemvParams &P, const float *xs
     for (int q = 0; q < 4; q++) dig[(b * 4 + q) * 8 + j] = pl[q];
     if (j == 0) {
       exps[b] = e;
-      units[b] = mx < kInfBits ? 1.f : __int_as_float(0x7fc00000);
+      units[b] = finite_max(mx) ? 1.f : __int_as_float(0x7fc00000);
     }
   }
   __syncthreads();
@@ -669,9 +669,9 @@ __global__ __launch_bounds__(kGemvThreads) void k_gemv_mma(GemvParams P) {
     for (int it = threadIdx.x; it < NB * 8; it += kGemvThreads) {
       const int b = it >> 3, j = it & 7;  // chunk j: elements 4j .. 4j+3
       const float4 v = *reinterpret_cast<const float4 *>(P.x + 32 * b + 4 * j);
-      const uint32_t mx = block_abs_bits(v);
+      const float mx = block_max_abs(v);
       int e = 0;
-      (void)frexpf(__uint_as_float(mx), &e);
+      (void)frexpf(mx, &e);
       const float xv[4] = {v.x, v.y, v.z, v.w};
       uint32_t pl[4] = {0u, 0u, 0u, 0u};
       int ps[4] = {0, 0, 0, 0};
@@ -704,7 +704,7 @@ __global__ __launch_bounds__(kGemvThreads) void k_gemv_mma(GemvParams P) {
         // the block's exponent, and 1 (NaN for a non-finite x: the rows'
         // sums then are NaN)
         exps[b] = e;
-        units[b] = mx < kInfBits ? 1.f : __int_as_float(0x7fc00000);
+        units[b] = finite_max(mx) ? 1.f : __int_as_float(0x7fc00000);
 #pragma unroll
         for (int q = 0; q < 4; q++) dsum[b * 4 + q] = ps[q];
       }

@@ -349,22 +349,22 @@ __global__ __launch_bounds__(kThreads) void k_wide(DecodeParams P, int z0) {
     } else {
       // make_digits' digits: a block's largest |q| over its lanes (eight of
       // a, eight of b; LLaMA: four of both)
-      uint32_t ma = 0u, mb = 0u;
+      float ma = 0.f, mb = 0.f;
 #pragma unroll
       for (int j = 0; j < 4; j++) {
-        ma = max(ma, abs_bits(a[j]));
-        mb = max(mb, abs_bits(b[j]));
+        ma = max_abs(ma, a[j]);
+        mb = max_abs(mb, b[j]);
       }
-      if (llama) ma = mb = max(ma, mb);
-      ma = max(ma, dpp_u<0xB1>(ma));
-      mb = max(mb, dpp_u<0xB1>(mb));
-      ma = max(ma, dpp_u<0x4E>(ma));
-      mb = max(mb, dpp_u<0x4E>(mb));
+      if (llama) ma = mb = max_abs(ma, mb);
+      ma = max_abs(ma, dpp_f<0xB1>(ma));
+      mb = max_abs(mb, dpp_f<0xB1>(mb));
+      ma = max_abs(ma, dpp_f<0x4E>(ma));
+      mb = max_abs(mb, dpp_f<0x4E>(mb));
       if (!llama) {
-        ma = max(ma, dpp_u<0x141>(ma));
-        mb = max(mb, dpp_u<0x141>(mb));
+        ma = max_abs(ma, dpp_f<0x141>(ma));
+        mb = max_abs(mb, dpp_f<0x141>(mb));
       }
-      auto put = [&](const f32x4 &x, uint32_t mx, int e) {
+      auto put = [&](const f32x4 &x, float mx, int e) {
         const DigitScale ds = digit_scale(mx);
         uint32_t d[kQPlanes] = {0u, 0u, 0u, 0u};
 #pragma unroll
