@@ -77,7 +77,7 @@ struct g2b_ctx {
   int32_t wq_dirty[2] = {0, 0};  // units of each set a launch may have left non-zero
   bool wq_reset = false;         // a launch failed after using the counters
   int32_t tune_stage = 0;      // -1: k_layer loads straight from HBM; 1, 2: staging mode
-  int32_t tune_kernel = 0;     // 0 automatic, 1 k_layer only, 2 k_tiles, 3 spanned k_short
+  int32_t tune_kernel = 0;     // 0 automatic, 1 k_layer only, 2 k_tiles, 3 spanned k_short, 4 k_wide
   int32_t *span_ctr = nullptr; // k_short's span tickets (zero between launches)
   size_t span_ctr_cap = 0;
   int32_t occ_wide = 0;           // k_wide workgroups per CU

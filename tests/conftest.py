@@ -13,6 +13,17 @@ def pytest_configure(config):
     config.addinivalue_line("markers", "gpu: needs an MI355X (gfx950) GPU")
 
 
+def pytest_collection_modifyitems(items):
+    """Tests that need the compiled reference run last: where it cannot be
+    built they fail (helpers.require_ref), and a run that stops at the first
+    failure has then run everything else."""
+    def needs_ref(item):
+        code = getattr(getattr(item, "function", None), "__code__", None)
+        return code is not None and "require_ref" in code.co_names + code.co_varnames
+
+    items.sort(key=needs_ref)
+
+
 @pytest.fixture(scope="session")
 def gpu_device():
     """Device 0, or skip when this host has no GPU (the CPU build container)."""
