@@ -295,29 +295,31 @@ struct QDigits {
 };
 
 // The digits of m (|m| <= 2^30): planes 0..2 in [-128, 127], plane 3 the
-// rest (|d3| <= 64).
+// rest (|d3| <= 64).  (Modulo 2^32: m is any int for a non-finite q.)
 __device__ __forceinline__ void split_digits(int m, int (&d)[kQPlanes]) {
 #pragma unroll
   for (int p = 0; p < kQPlanes - 1; p++) {
-    d[p] = ((m + 128) & 255) - 128;
-    m = (m - d[p]) >> 8;
+    d[p] = (int)(((uint32_t)m + 128u) & 255u) - 128;
+    m = (int)((uint32_t)m - (uint32_t)d[p]) >> 8;
   }
   d[kQPlanes - 1] = m;
 }
 
 // 2^(kQBits-e) and 2^(e-kQBits) of a chunk whose largest |q| (max_abs) is mx.
-// A chunk that holds an Inf or a NaN has no digits: they are 0
-// and the unit is NaN, so every score of its head, and with them the head's
-// output, is NaN, as in the fp32 dot (Inf in q meets both signs of k; the
-// softmax of infinite scores is NaN).
+// The digits of a chunk that holds an Inf or a NaN say nothing and its unit is
+// NaN (mx - mx is, else 0), so every score of its head, and with them the
+// head's output, is NaN, as in the fp32 dot (Inf in q meets both signs of k;
+// the softmax of infinite scores is NaN).  Not a select on mx: with one, the
+// compiler had the work queue's visits wait for the staged chunk in the middle
+// of the setup (32 sequences of 643 positions, 16 / 8 heads of 128: 47.8 us
+// instead of 43.4).
 struct DigitScale {
   float up, unit;
 };
 __device__ __forceinline__ DigitScale digit_scale(float mx) {
   int e = 0;
   (void)frexpf(mx, &e);
-  if (!finite_max(mx)) return {0.f, __int_as_float(0x7fc00000)};
-  return {ldexpf(1.f, kQBits - e), ldexpf(1.f, e - kQBits)};
+  return {ldexpf(1.f, kQBits - e), ldexpf(1.f, e - kQBits) + (mx - mx)};
 }
 
 template <int CD>
