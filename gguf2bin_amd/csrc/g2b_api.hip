@@ -279,24 +279,59 @@ int64_t unit_positions(int32_t max_pos) {
 // to spare: 8 sequences of 1000-4000, 2 KV heads of 8 q heads, 16.6 us in 592
 // of 96 (19.4 in 896 of 64, 20.5 in 720 of 80, 17.2 in 448 of 128, 17.0 in 224
 // of 256).
+//
+// On some of k_layer's shapes a batch's cut differs, where the one above loses to
+// k_layer (us per call; 32-bit errors relative to 64 bits).
+//  - Q8_0 rows that are not whole 16-byte pieces (k_layer reads them per lane),
+//    more than 64 units shorter than k_layer's own shortest split (it writes the
+//    output itself there): the whole context.  9 / 3 heads of 64, 256 sequences of
+//    7-143 positions 20.8 in two splits -> 10.3 (k_layer 11.9), 96 12.3 in three ->
+//    8.2; of 140-143 12.9 (k_layer 12.3).  Error 9.4e-8 at 7-143 (splits of 64
+//    1.0e-7, k_layer 1.6e-7), 6.7e-8 at 143 (6.3e-8, 1.1e-7).
+//  - those rows, 9 to 12 splits: 8 or fewer.  The grid has a multiple of eight per
+//    sequence (launch_wide_sets), so nine start sixteen, which costs once these
+//    are more than three workgroups per CU: 32 sequences of 803 15.7 in nine
+//    splits of 96 -> 12.2 in eight of 112 (k_layer 13.9), one sequence x 28 layers
+//    of 803 15.7 -> 12.8 (14.5).  With fewer workgroups more splits win: 2
+//    sequences of 643 8.8 in ten of 64, 10.2 in eight of 80.
+//  - F32, 1 q head of 64 per KV head, below 512 positions, two splits: the whole
+//    context.  8 / 8 heads, 64 sequences of 150-303 25.4 in two -> 14.1 (k_layer
+//    19.9), 40 of 303 16.3 -> 13.6.  Error 6.8e-8 (two 6.8e-8, k_layer 6.9e-8) at
+//    150-303, 6.1e-8 (6.1e-8, 6.0e-8) at 250-503, 8.9e-8 (9.3e-8, 9.3e-8) at 15-303.
+// Everywhere else the finer cut has the smaller error.  Over 12 shapes, 2 to 256
+// units, 140 to 8000 positions, uniform and ragged (7875 calls that wide_latency
+// gives to k_wide) 49 are more than 2% behind k_layer or k_tiles, 32 more than 5%,
+// at most 20% (40 sequences of 25-503, 4 / 4 heads of 128, F32, 22.5 against 18.7;
+// 8 of 150-3003, 8 / 8 of 64, Q8_0, 18.9 against 16.1; 192 of 203, 9 / 3 of 64,
+// Q8_0, 20.2 against 18.3); the mean of the ratios is 0.53.
 constexpr int32_t kWideWhole = 128;
 int32_t wide_split(const g2b_ctx *c, int64_t slots, int32_t n_seq, int64_t total_pos,
                    int32_t max_pos, int32_t n_layers) {
   const int64_t units = (int64_t)n_seq * n_layers, nkvh = c->shape.n_kv_heads;
+  const bool layer_shape = decode_fast_available(c->sh);
+  const bool unstaged = layer_shape && c->sh.kv_q8 && (c->sh.row_bytes & 15u);
+  const bool f32_64 = layer_shape && !c->sh.kv_q8 && c->sh.head_dim == 64 &&
+                      c->sh.n_heads == c->sh.n_kv_heads && max_pos < 512;
   int64_t sl;
-  if (max_pos < kWideWhole) {
-    sl = kWideWhole;
+  if (max_pos < kWideWhole ||
+      (unstaged && units > 64 && max_pos < kWavesPerSplit * 8 * decode_ppw(c->sh, 0))) {
+    sl = (int64_t)max_pos + 1;
   } else if (units == 1) {
     const int64_t splits = std::max<int64_t>(slots / nkvh, 1);
     sl = (unit_positions(max_pos) + splits * kWideRound - 1) / (splits * kWideRound) * kWideRound;
   } else {
     const int64_t splits = std::max<int64_t>(slots * 9 / 10 / nkvh - units / 2, 1);
-    sl = ((total_pos * n_layers + splits - 1) / splits + 15) / 16 * 16;
+    sl = std::max<int64_t>(((total_pos * n_layers + splits - 1) / splits + 15) / 16 * 16,
+                           kWideRound);
+    const int64_t x = (max_pos + sl) / sl;
+    if (unstaged && x > 8 && x <= 12 && units * nkvh * 16 > 3 * std::max(1, c->n_cu))
+      sl = ((max_pos + 8) / 8 + 15) / 16 * 16;
+    if (f32_64 && x == 2) sl = (int64_t)max_pos + 1;
   }
   sl = std::max<int64_t>(sl, kWideRound);
   if (c->split_override > 0) sl = c->split_override;
   sl = std::max(sl, ((int64_t)max_pos + 512) / 512);
-  if (!decode_fast_available(c->sh)) sl = std::min<int64_t>(sl, kGenericMaxSplit);
+  if (!layer_shape) sl = std::min<int64_t>(sl, kGenericMaxSplit);
   return (int32_t)std::min<int64_t>(sl, (int64_t)max_pos + 1);
 }
 
@@ -327,20 +362,14 @@ int32_t wide_split(const g2b_ctx *c, int64_t slots, int32_t n_seq, int64_t total
 //    longer streams win (4 of 1500-3003, F32, 74 MB 24.0 -> 25.5; 64 of 750-1503,
 //    9 / 3, Q8_0, 29 MB 23.4 -> 25.5).  k_tiles has the longest setup: 16 of
 //    1000-2003, 32 / 8, Q8_0 (52 MB) 34.5 -> 29.0, 32 of 500-999 (52 MB) 68.8 ->
-//    29.5, 64 of 750-1503 (157 MB) 70.5 -> 101.6.  Not 33 to 47 units (21 to
-//    47 in a call over several layers), which within 16 MiB have 512 positions
-//    only where rows are short (9 / 3 of 64, Q8_0): there k_layer's splits end
-//    evenly and k_wide's do not: 40 sequences of 350-703 15.2 -> 16.9, of
-//    600-1203 17.2 -> 19.1 (of 450-903 18.0 -> 14.0); 32 of 350-703 15.2 -> 14.6,
-//    of 600-1203 16.9 -> 16.6, 28 15.9 -> 16.1, 48 of 350-703 15.2 -> 14.4.
+//    29.5, 64 of 750-1503 (157 MB) 70.5 -> 101.6.
 // Calls over several layers turn at the same lines (us per call, before ->
 // k_wide): below kWideWhole, 1 sequence x 28 layers of 47 9.0 -> 6.7, 64 x 28 of
 // 50-103 186 -> 150, F32 8 x 28 of 50-103 (141 MB) 33.7 -> 34.5, 64 x 4 (172 MB)
 // 39.7 -> 37.9; 1 x 28 of 503 20.4 -> 18.8, 2 x 28 of 250-503 57.0 -> 33.6, 32 / 8
 // 2 x 32 57.8 -> 23.6; 1 x 8 of 903 18.5 -> 16.5, 32 / 8 8 x 4 of 500-1003 (52
-// MB) 67.6 -> 26.9; 9 / 3, Q8_0, 1 x 20 of 1203 14.6 -> 13.1, 2 x 30 of 350-703
-// 17.3 -> 15.6, but 1 x 24 of 1203 14.8 -> 15.7, 1 x 30 of 1003 13.9 -> 16.0, 4 x 8
-// of 400-803 15.1 -> 16.1, 20 x 2 of 350-703 15.3 -> 17.1.
+// MB) 67.6 -> 26.9; 9 / 3, Q8_0, 1 x 20 of 1203 14.6 -> 13.1, 1 x 30 of 1003 14.0
+// -> 12.9, 20 x 2 of 350-703 15.5 -> 13.6.
 bool wide_latency(const ShapeDev &sh, int32_t n_seq, int32_t n_layers, int32_t max_pos,
                   int64_t total_pos) {
   constexpr int64_t kMiB = 1 << 20;
@@ -349,9 +378,10 @@ bool wide_latency(const ShapeDev &sh, int32_t n_seq, int32_t n_layers, int32_t m
   const bool t = tiles_available(sh), f32_4k = !sh.kv_q8 && sh.row_bytes >= 4096;
   if (max_pos < kWideWhole) return !f32_4k || bytes <= 160 * kMiB;
   if (units == 1) return !t || unit_positions(max_pos) <= 16384;
-  if (units <= 64 && max_pos < 512) return !f32_4k || bytes <= 32 * kMiB;
+  if (units <= 64 && max_pos < 512)
+    return !f32_4k || bytes <= 32 * kMiB;
   if (t) return bytes <= 52 * kMiB;
-  return bytes <= 16 * kMiB && (units <= (n_layers == 1 ? 32 : 20) || units >= 48);
+  return bytes <= 16 * kMiB;
 }
 
 // Positions per split of a static schedule of k_layer, k_tiles or the generic

@@ -44,7 +44,7 @@
 // so that no window leaves the row.  Neighbouring windows share lines, which
 // the vector cache serves (default policy), and so do neighbouring KV heads of
 // a row (136 bytes each): the grid puts the KV heads of a split on one XCD
-// (wide_grid), whose L2 then fetches each line once.
+// (launch_wide_sets), whose L2 then fetches each line once.
 //
 // What bounds it: HBM in large batches, else that chain.  Measured per layer
 // against the three-pass kernel that wide groups took before (one thread per

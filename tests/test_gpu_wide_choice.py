@@ -1,5 +1,5 @@
-"""Which calls of k_layer's shapes the automatic choice gives to k_wide, on
-both sides of each line of the rule, against the oracle."""
+"""Which calls of k_layer's shapes the automatic choice gives to k_wide, and in
+how many splits, on both sides of each line of the rule, against the oracle."""
 from __future__ import annotations
 
 import pytest
@@ -13,9 +13,11 @@ SHAPES = {
     "qwen3_q8": (16, 8, 128, orc.ARCH_QWEN3, True),
     "qwen3_f32": (16, 8, 128, orc.ARCH_QWEN3, False),
     "smollm2_q8": (9, 3, 64, orc.ARCH_LLAMA, True),
+    "smollm2_f32": (9, 3, 64, orc.ARCH_LLAMA, False),
     "llama3_q8": (32, 8, 128, orc.ARCH_LLAMA, True),
+    "mha_f32": (8, 8, 64, orc.ARCH_LLAMA, False),
 }
-# shape, positions, weights output, kernel[, layers in the one call]
+# shape, positions, weights output, kernel[, layers in the one call[, splits]]
 CASES = [
     ("qwen3_q8", [127], False, "k_wide"),
     ("qwen3_q8", [700], False, "k_wide"),
@@ -29,14 +31,24 @@ CASES = [
     ("qwen3_f32", [8192], False, "k_wide"),
     ("llama3_q8", [16383], False, "k_wide"),
     ("llama3_q8", [16384], False, "k_tiles"),
-    # units of up to 513 positions of 408 bytes: 20 and 21 in a call over several
-    # layers, 32, 33, 47 and 48 in one layer
-    ("smollm2_q8", [512, 64], False, "k_wide", 10),
-    ("smollm2_q8", [512, 64, 31], False, "k_layer", 7),
-    ("smollm2_q8", [512] + [40] * 31, False, "k_wide"),
-    ("smollm2_q8", [512] + [40] * 32, False, "k_layer"),
-    ("smollm2_q8", [512] + [40] * 46, False, "k_layer"),
-    ("smollm2_q8", [512] + [40] * 47, False, "k_wide"),
+    # rows of 204 bytes, more than 64 units below k_layer's shortest split (160):
+    # the whole context in one split that writes the output
+    ("smollm2_q8", [159] + [40] * 64, False, "k_wide", 1, 1),
+    ("smollm2_q8", [159] + [40] * 63, False, "k_wide", 1, 3),
+    ("smollm2_q8", [160] + [40] * 64, False, "k_wide", 1, 3),
+    ("smollm2_q8", [128, 159, 7, 40, 97], False, "k_wide", 14, 1),
+    ("smollm2_f32", [159] + [40] * 64, False, "k_wide", 1, 3),
+    # rows of 204 bytes: nine to twelve splits become eight or fewer (whole tiles
+    # of 16) once sixteen per unit are more than three workgroups per CU
+    ("smollm2_q8", [640] * 16, False, "k_wide", 1, 11),
+    ("smollm2_q8", [640] * 17, False, "k_wide", 1, 7),
+    ("smollm2_q8", [800] * 24, False, "k_wide", 1, 8),
+    ("smollm2_q8", [703], False, "k_wide", 28, 8),
+    ("smollm2_f32", [640] * 17, False, "k_wide", 1, 11),
+    # one F32 q head of 64 per KV head, below 512 positions: two splits become one
+    ("mha_f32", [303] * 20 + [150] * 44, False, "k_wide", 1, 1),
+    ("mha_f32", [511] + [300] * 63, False, "k_wide", 1, 1),
+    ("mha_f32", [303] + [15] * 20, False, "k_wide", 1, 5),
     # rows of 4 KB, F32: 163840 KB of positions below 128 in one call are the line
     ("qwen3_f32", [127] * 5, False, "k_wide", 32),
     ("qwen3_f32", [127] * 5 + [0], False, "k_short", 32),
@@ -47,6 +59,7 @@ CASES = [
     [c[0], f"{len(c[1])}x{max(c[1])}", *map(str, c[2:])]))
 def test_choice(gpu_device, case):
     (name, poss, att, kernel), layers = case[:4], case[4] if len(case) > 4 else 1
+    splits = case[5] if len(case) > 5 else None
     nh, nkv, hd, arch, q8 = SHAPES[name]
     o = orc.Shape(layers, nh, nkv, hd, 1e5, arch, q8)
     # (rows of 204 bytes: whole capacities of eight rows keep caches aligned)
@@ -55,3 +68,6 @@ def test_choice(gpu_device, case):
     sched = {}
     run_batch_case(o, caps, poss, seed=71, fused=layers > 1, want_att=att, sched=sched)
     assert sched["kernel"] == kernel and sched["variant"].startswith(kernel + "<"), sched
+    if splits:
+        assert sched["max_splits"] == splits, sched
+        assert sched["output_in_kernel"] == (splits == 1), sched
